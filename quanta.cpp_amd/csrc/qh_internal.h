@@ -171,6 +171,23 @@ hipError_t launch_sample(const float* logits, int n_valid, const int32_t* rows, 
                          const HeadMust& hist, const qh_sampler_params& p, uint64_t* state, int32_t* out_id,
                          void* ws, hipStream_t s);
 
+// Attention of a prefill stack over the f16 cache (qh_attn.hip): n tokens at positions pos0 .., their projections q
+// [n][n_heads * head_dim] (without bias or RoPE), every cache row up to pos0 + n stored; one layer's kc / vc in the
+// decoder's layouts; the outputs quantized to oq / od (and f32 to of when given).
+// The members after `of` belong to the launch.
+struct AttnStack {
+    const float *q, *bq, *cs;
+    const uint16_t *kc, *vc;
+    int ctx, n_heads, n_kv, n, pos0;
+    int8_t* oq;
+    float *od, *of;
+    int rs;              // workspace rows per pair group
+    float *s, *pm, *inv;  // scores [n_kv * groups][rs / 4][64][4], maxima, inverse sums
+};
+constexpr size_t kAttnWsBytes = (size_t)256 << 20;
+size_t attn_stack_ws_bytes(int n_heads, int n_kv, int ctx, int tokens);
+hipError_t launch_attention_stack(AttnStack a, int head_dim, float* ws, size_t ws_bytes, hipStream_t s);
+
 // GPU-resident decoder (qh_decoder.hip). Tensors in qh_decoder_create order; all sizes validated by the caller.
 struct Decoder;
 int decoder_create(const qh_model_desc* hp, const qh_tensor* tensors, int n_tensors, Decoder** out);
