@@ -228,7 +228,7 @@ __global__ __launch_bounds__(64 * kSoftWaves) void attn_softmax_kernel(AttnStack
                 float e[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    e[i] = dev_expf(x[i] - mx, exptab);
+                    e[i] = dev_expf_nonpos(x[i] - mx, exptab);
                     e[i] = 16 * bg + 4 * i + (lane >> 4) < rows ? e[i] : 0.0f;  // +0 leaves a pair's sum as it is
                 }
                 const float4 v = make_float4(e[0], e[1], e[2], e[3]);
@@ -545,7 +545,7 @@ __global__ __launch_bounds__(256) void attn_short_kernel(AttnStack a, int ng16) 
         float e[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            e[t] = dev_expf(e[t] - mx, exptab);
+            e[t] = dev_expf_nonpos(e[t] - mx, exptab);
             e[t] = 16 * b + 4 * t + lq < rows ? e[t] : 0.0f;  // +0 leaves a pair's sum as it is
         }
         es[64 * b + lane] = make_float4(e[0], e[1], e[2], e[3]);
@@ -585,39 +585,35 @@ __global__ __launch_bounds__(256) void attn_short_kernel(AttnStack a, int ng16) 
     for (int d = 0; d < DT; ++d) acc[d] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
     const int steps = lo / 4;  // of 4 positions that are rows of every pair
     float4 x = es[lane];
-    for (int b0 = 0; 4 * b0 < steps; b0 += kAhead) {
+    auto block = [&](auto full, int u, int b) {
+        const float p[4] = {x.x * inv, x.y * inv, x.z * inv, x.w * inv};
+        float vf[DT][4];
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u) {
-            const int b = b0 + u, n = steps - 4 * b;
-            const float p[4] = {x.x * inv, x.y * inv, x.z * inv, x.w * inv};
-            float vf[DT][4];
+        for (int d = 0; d < DT; ++d)
 #pragma unroll
-            for (int d = 0; d < DT; ++d)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    uint32_t w[4] = {v[u].w[d][h][0], v[u].w[d][h][1], v[u].w[d][h][2], v[u].w[d][h][3]};
-                    asm("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
-                    vf[d][2 * h] = half(second ? w[1] : w[0]);
-                    vf[d][2 * h + 1] = half(second ? w[3] : w[2]);
-                }
-            v[u] = vload(b + kAhead);
-            x = es[64 * min(b + 1, nb - 1) + lane];
-            __builtin_amdgcn_sched_barrier(0);
-            if (n >= 4) {  // uniform
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int d = 0; d < DT; ++d) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[t], vf[d][t], acc[d], 0, 0, 0);
-            } else {
-#pragma unroll
-                for (int t = 0; t < 3; ++t)
-                    if (t < n)
-#pragma unroll
-                        for (int d = 0; d < DT; ++d) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[t], vf[d][t], acc[d], 0, 0, 0);
+            for (int h = 0; h < 2; ++h) {
+                uint32_t w[4] = {v[u].w[d][h][0], v[u].w[d][h][1], v[u].w[d][h][2], v[u].w[d][h][3]};
+                asm("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
+                vf[d][2 * h] = half(second ? w[1] : w[0]);
+                vf[d][2 * h + 1] = half(second ? w[3] : w[2]);
             }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
+        v[u] = vload(b + kAhead);
+        x = es[64 * min(b + 1, nb - 1) + lane];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (decltype(full)::value || 4 * b + t < steps)  // uniform
+#pragma unroll
+                for (int d = 0; d < DT; ++d) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[t], vf[d][t], acc[d], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int vbk = 0;
+    for (; 4 * (vbk + kAhead) <= steps; vbk += kAhead)
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) block(std::true_type{}, u, vbk + u);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+        if (4 * (vbk + u) < steps) block(std::false_type{}, u, vbk + u);  // uniform
     // The rows past the first pair's whole steps, for the pairs that have them (a later token's row is not an earlier
     // one's, and 0 times an infinite value is not 0): lane l's pairs 4 lq + i.
     for (int j = 4 * steps; j < hi; ++j) {
