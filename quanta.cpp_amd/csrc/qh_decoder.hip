@@ -2343,6 +2343,22 @@ hipError_t linear(Decoder* d, float* out, int ldo, const qh_tensor& W, bool inne
     return launch_matmul(out, ldo, W, xq, xd, n, 0, W.rows, s);
 }
 
+// linear() of up to three matrices over one activation, the unquantized ones of one dtype that follow one another in one
+// launch.
+hipError_t linear_group(Decoder* d, const MmOut* m, int k, bool inner, int n, hipStream_t s) {
+    for (int i = 0; i < k;) {
+        int j = i + 1;
+        if (dense_w(*m[i].W)) {
+            while (j < k && m[j].W->dtype == m[i].W->dtype && m[j].W->cols == m[i].W->cols) ++j;
+            QH_TRY(launch_dense_segs(m + i, j - i, inner ? d->fb : d->fa, m[i].W->cols, n, nullptr, s));
+        } else {
+            QH_TRY(linear(d, m[i].out, m[i].ldo, *m[i].W, inner, n, s));
+        }
+        i = j;
+    }
+    return hipSuccess;
+}
+
 // The normed-input fill of a decode kernel: layer input from the residual stream x, or (first layer) from the
 // embedding of the current token, which workgroup 0 also stores as x.
 NormAct make_norm(Decoder* d, bool embedding, const float* w) {
@@ -2407,9 +2423,8 @@ hipError_t residual(Decoder* d, const qh_tensor& W, hipStream_t s) {
     const int8_t* xq = d->qb;
     const float* xd = d->db;
     if (dense_w(W)) {
-        QH_TRY(linear(d, d->o, 0, W, true, 1, s));
-        qh_launch(residual_add_kernel, dim3((unsigned)((W.rows + 255) / 256)), dim3(256), 0, s, d->x, d->o, W.rows);
-        return hipGetLastError();
+        const MmOut m{&W, d->x, 0, 0, W.rows};
+        return launch_dense_segs(&m, 1, d->fb, W.cols, 1, d->x, s);
     }
     const GemvPlan p = gemv_plan(W.dtype, W.cols, W.rows);
     if (d->fuse && !p.stream) {
@@ -2471,8 +2486,8 @@ hipError_t gate_up(Decoder* d, int l, hipStream_t s) {
         return hipGetLastError();
     }
     QH_TRY(norm_quant(d, lf(d, l, L_FFN_NORM), d->fa, s));
-    QH_TRY(linear(d, d->g, 0, wg, false, 1, s));
-    QH_TRY(linear(d, d->u, 0, wu, false, 1, s));
+    const MmOut m[2] = {{&wg, d->g, 0, 0, wg.rows}, {&wu, d->u, 0, 0, wu.rows}};
+    QH_TRY(linear_group(d, m, 2, false, 1, s));
     return swiglu_down_input(d, wg.rows, 1, s);
 }
 
@@ -2577,9 +2592,9 @@ hipError_t decode_layers(Decoder* d, hipStream_t s) {
                 QH_TRY(embed(d, d->tokens, 1, s));
             else
                 QH_TRY(norm_quant(d, lf(d, l, L_ATTN_NORM), d->fa, s));
-            QH_TRY(linear(d, d->q, 0, lt(d, l, L_WQ), false, 1, s));
-            QH_TRY(linear(d, d->k, 0, lt(d, l, L_WK), false, 1, s));
-            QH_TRY(linear(d, d->v, 0, lt(d, l, L_WV), false, 1, s));
+            const qh_tensor &wq = lt(d, l, L_WQ), &wk = lt(d, l, L_WK), &wv = lt(d, l, L_WV);
+            const MmOut m[3] = {{&wq, d->q, 0, 0, wq.rows}, {&wk, d->k, 0, 0, wk.rows}, {&wv, d->v, 0, 0, wv.rows}};
+            QH_TRY(linear_group(d, m, 3, false, 1, s));
         }
         d->mark(l * QH_STAGES_PER_LAYER + QH_STAGE_QKV);
         QH_TRY(attention(d, l, 1, s));
@@ -2656,7 +2671,7 @@ hipError_t prefill_layers(Decoder* d, int n, hipStream_t s) {
         const MmOut qkv[3] = {{&wq, d->q, wq.rows, 0, wq.rows}, {&wk, d->k, wk.rows, 0, wk.rows},
                               {&wv, d->v, wv.rows, 0, wv.rows}};
         if (dense_w(wq) || dense_w(wk) || dense_w(wv)) {
-            for (const MmOut& m : qkv) QH_TRY(linear(d, m.out, m.ldo, *m.W, false, n, s));
+            QH_TRY(linear_group(d, qkv, 3, false, n, s));
         } else {
             QH_TRY(matmul_group(qkv, 3, d->qa, d->da, n, s));
         }
@@ -2678,7 +2693,7 @@ hipError_t prefill_layers(Decoder* d, int n, hipStream_t s) {
         } else if (!swiglu_fused(d, wg, wu, n, s)) {
             const MmOut gu[2] = {{&wg, d->g, wg.rows, 0, wg.rows}, {&wu, d->u, wu.rows, 0, wu.rows}};
             if (dense_w(wg) || dense_w(wu)) {
-                for (const MmOut& m : gu) QH_TRY(linear(d, m.out, m.ldo, *m.W, false, n, s));
+                QH_TRY(linear_group(d, gu, 2, false, n, s));
             } else {
                 QH_TRY(matmul_group(gu, 2, d->qa, d->da, n, s));
             }

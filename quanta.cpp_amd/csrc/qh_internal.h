@@ -82,6 +82,9 @@ struct MmOut {
     float* out;
     int ldo, r0, r1;
 };
+// matvec_ref over up to three F32 / F16 matrices of one dtype and width, one launch (q / k / v, gate / up); res (one
+// token, one matrix): out[r] = res[r] + W[r,:] . x.
+hipError_t launch_dense_segs(const MmOut* m, int n_mats, const float* x, int ldx, int n, const float* res, hipStream_t s);
 // Up to three matrices of one dtype and width over the same activation in one launch (prefill q / k / v, gate / up).
 hipError_t launch_matmul_segs(const MmOut* m, int n_mats, const int8_t* xq, const float* xd, int n, hipStream_t s);
 // Gate / up of n >= 128 tokens (a prefill stack) with h = g / (1 + expf(-g)) * u quantized per 32 rows into hq / hd
