@@ -109,22 +109,6 @@ __device__ __forceinline__ float wave_max_sel(float a) {
     return step(__builtin_bit_cast(float, (uint32_t)s32[0]), __builtin_bit_cast(float, (uint32_t)s32[1]));
 }
 
-// The same for a block held four consecutive values per lane by an aligned group of 8 lanes (lane j of the group
-// holds elements 4j .. 4j + 3): one 4-byte store of codes per lane.
-__device__ __forceinline__ void quant_block_x8(float4 v, int8_t* __restrict__ q, float* __restrict__ d) {
-    const float a = max8_lanes(__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(v.x), __builtin_fabsf(v.y)),
-                                               __builtin_fmaxf(__builtin_fabsf(v.z), __builtin_fabsf(v.w))));
-    const float sc = a / 127.0f;
-    const float inv = sc > 0.0f ? 1.0f / sc : 0.0f;
-    const int j = (int)threadIdx.x & 7;
-    const uint32_t c0 = (uint32_t)(uint8_t)(int8_t)(int)round_half_away(v.x * inv);
-    const uint32_t c1 = (uint32_t)(uint8_t)(int8_t)(int)round_half_away(v.y * inv);
-    const uint32_t c2 = (uint32_t)(uint8_t)(int8_t)(int)round_half_away(v.z * inv);
-    const uint32_t c3 = (uint32_t)(uint8_t)(int8_t)(int)round_half_away(v.w * inv);
-    *reinterpret_cast<uint32_t*>(q + 4 * j) = c0 | (c1 << 8) | (c2 << 16) | (c3 << 24);
-    if (j == 0) *d = sc;
-}
-
 // quantize_q8 of the row xs[0, D) (16-byte aligned, D % 32 == 0) into q / d: 8 lanes per block, 32 blocks per pass
 // of 256 threads.
 __device__ __forceinline__ void quant_row_x8(const float* xs, int D, int8_t* __restrict__ q, float* __restrict__ d) {

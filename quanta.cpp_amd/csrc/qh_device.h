@@ -345,4 +345,20 @@ __device__ __forceinline__ void quant_block32(float v, int8_t* __restrict__ q, f
     if (i == 0) *d = sc;
 }
 
+// The same for a block held four consecutive values per lane by an aligned group of 8 lanes (lane j of the group
+// holds elements 4j .. 4j + 3): one 4-byte store of codes per lane.
+__device__ __forceinline__ void quant_block_x8(float4 v, int8_t* __restrict__ q, float* __restrict__ d) {
+    const float a = max8_lanes(__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(v.x), __builtin_fabsf(v.y)),
+                                               __builtin_fmaxf(__builtin_fabsf(v.z), __builtin_fabsf(v.w))));
+    const float sc = a / 127.0f;
+    const float inv = sc > 0.0f ? 1.0f / sc : 0.0f;
+    const int j = (int)threadIdx.x & 7;
+    const uint32_t c0 = (uint32_t)(uint8_t)(int8_t)(int)round_half_away(v.x * inv);
+    const uint32_t c1 = (uint32_t)(uint8_t)(int8_t)(int)round_half_away(v.y * inv);
+    const uint32_t c2 = (uint32_t)(uint8_t)(int8_t)(int)round_half_away(v.z * inv);
+    const uint32_t c3 = (uint32_t)(uint8_t)(int8_t)(int)round_half_away(v.w * inv);
+    *reinterpret_cast<uint32_t*>(q + 4 * j) = c0 | (c1 << 8) | (c2 << 16) | (c3 << 24);
+    if (j == 0) *d = sc;
+}
+
 }  // namespace qh
