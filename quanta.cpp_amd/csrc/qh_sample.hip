@@ -51,17 +51,61 @@ __device__ uint64_t block_max_u64(uint64_t v, uint64_t* red) {
 
 }  // namespace
 
+// The largest key of each group of kGroup ids (every id below n_valid a candidate), 4 groups to a workgroup.
+constexpr int kGroup = 256, kGroupThreads = 256;
+__global__ __launch_bounds__(kGroupThreads) void sample_groups_kernel(const float* __restrict__ logits, int n_valid,
+                                                                      HeadMust hist, float penalty,
+                                                                      uint64_t* __restrict__ gmax) {
+    constexpr int kIds = kGroup * kGroupThreads / 64;
+    __shared__ uint32_t seen[kIds / 32];
+    const int tid = (int)threadIdx.x, first = (int)blockIdx.x * kIds;
+    float l[kGroup / 64];
+    const int id0 = first + (tid >> 6) * kGroup + (tid & 63);
+#pragma unroll
+    for (int j = 0; j < kGroup / 64; ++j) l[j] = logits[min(id0 + 64 * j, n_valid - 1)];
+    if (penalty != 1.0f) {
+        if (tid < kIds / 32) seen[tid] = 0u;
+        __syncthreads();
+        const int32_t* h;
+        int nh;
+        must_span(hist, h, nh);
+        for (int i = tid; i < nh; i += kGroupThreads) {
+            const int at = h[i] - first;
+            if (at >= 0 && at < kIds) atomicOr(&seen[at >> 5], 1u << (at & 31));
+        }
+        __syncthreads();
+    }
+    uint64_t m = 0;
+#pragma unroll
+    for (int j = 0; j < kGroup / 64; ++j) {
+        const int id = id0 + 64 * j, at = id - first;
+        if (penalty != 1.0f && ((seen[at >> 5] >> (at & 31)) & 1u)) l[j] = l[j] > 0 ? l[j] / penalty : l[j] * penalty;
+        const uint64_t key = id < n_valid ? score_key(l[j], id) : 0ull;
+        m = key > m ? key : m;
+    }
+    m = wave_max_u64(m);
+    const int g = (int)blockIdx.x * (kGroupThreads / 64) + (tid >> 6);
+    if ((tid & 63) == 0 && g * kGroup < n_valid) gmax[g] = m;
+}
+
+// gmax: the groups' largest keys (n_groups of them, rows null), or null.
 __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restrict__ logits, int n_valid,
                                                           const int32_t* __restrict__ rows,
                                                           const qh_head_stats* __restrict__ hs, HeadMust hist,
                                                           qh_sampler_params p, uint64_t* __restrict__ state,
-                                                          int32_t* __restrict__ out_id) {
+                                                          int32_t* __restrict__ out_id,
+                                                          const uint64_t* __restrict__ gmax, int n_groups) {
     extern __shared__ uint32_t seen[];  // [ceil(n_valid / 32)]: history ids, when the penalty is on
     __shared__ uint64_t pool[kPool];
+    __shared__ int n_list;
+    __shared__ uint32_t ghi;
     __shared__ uint64_t red[kWaves];
     __shared__ uint64_t wbound[kWaves];
-    __shared__ float cval[QH_SAMPLE_MAX_TOPK];
-    __shared__ int cid[QH_SAMPLE_MAX_TOPK];
+    __shared__ uint32_t survivors[2 * QH_SAMPLE_MAX_TOPK];
+    float* cval = reinterpret_cast<float*>(survivors);
+    int* cid = reinterpret_cast<int*>(survivors + QH_SAMPLE_MAX_TOPK);
+    uint16_t* glist = reinterpret_cast<uint16_t*>(survivors);  // until the pool is filled: the groups to read
+    static_assert(kThreads * sizeof(uint16_t) <= sizeof(survivors), "a group per thread");
     __shared__ int pool_n;
     __shared__ float sum_sh;
     __shared__ uint64_t exptab[32];  // expf's table in LDS: the softmax below reads it without a cache round trip
@@ -91,9 +135,13 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
 
     if (p.temperature <= 0.0f) {  // first maximum (sampler.cpp:35-37)
         uint64_t m = 0;
-        for (int i = tid; i < n; i += kThreads) {
-            const uint64_t k = key_of(i);
-            m = k > m ? k : m;
+        if (gmax) {
+            if (tid < n_groups) m = gmax[tid];
+        } else {
+            for (int i = tid; i < n; i += kThreads) {
+                const uint64_t k = key_of(i);
+                m = k > m ? k : m;
+            }
         }
         m = block_max_u64(m, red);
         if (tid == 0) *out_id = m ? key_row(m) : 0;
@@ -107,7 +155,34 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
     // so for k <= 64 the first 64 entries already hold k candidates: each wave's k-th largest of its 64 bounds it.
     // Past 1024 candidates otherwise: the k-th largest of the threads' own maxima (k distinct candidates are at or
     // above it).
-    if (n > kThreads && (!rows || k > 64)) {
+    int nc = n;  // candidates to filter: all, or those of the listed groups
+    if (gmax) {
+        // The k-th largest group maximum bounds the k-th largest key from below, and only groups whose maximum reaches
+        // it hold larger ones: wave 0 finds the largest score bits T that at least k maxima reach, bit by bit.
+        const uint64_t mine = tid < n_groups ? gmax[tid] : 0ull;
+        pool[tid] = mine;
+        if (tid == 0) pool_n = n_list = 0;
+        __syncthreads();
+        if (wave == 0) {
+            uint32_t h[kWaves];
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) h[w] = (uint32_t)(pool[64 * w + lane] >> 32);
+            uint32_t t = 0u;
+            for (int bit = 31; bit >= 0; --bit) {
+                const uint32_t c = t | (1u << bit);
+                int at_least = 0;
+#pragma unroll
+                for (int w = 0; w < kWaves; ++w) at_least += (int)__popcll(__ballot(h[w] >= c));
+                t = at_least >= k ? c : t;
+            }
+            if (lane == 0) ghi = t;
+        }
+        __syncthreads();
+        thr = (uint64_t)ghi << 32;
+        if (mine != 0 && mine >= thr) glist[atomicAdd(&n_list, 1)] = (uint16_t)tid;
+        __syncthreads();
+        nc = n_list * kGroup;
+    } else if (n > kThreads && (!rows || k > 64)) {
         uint64_t m = 0;
 #pragma unroll 8
         for (int i = tid; i < n; i += kThreads) {
@@ -141,8 +216,9 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
     }
     thr = thr ? thr : 1ull;  // no bound: every real key (keys are nonzero)
 #pragma unroll 8
-    for (int i = tid; i < n; i += kThreads) {
-        const uint64_t key = key_of(i);
+    for (int c = tid; c < nc; c += kThreads) {
+        const int i = gmax ? glist[c / kGroup] * kGroup + c % kGroup : c;
+        const uint64_t key = i < n ? key_of(i) : 0ull;
         if (key >= thr) {
             const int at = atomicAdd(&pool_n, 1);
             if (at < kPool) pool[at] = key;
@@ -509,8 +585,18 @@ hipError_t launch_sample(const float* logits, int n_valid, const int32_t* rows, 
                          void* ws, hipStream_t s) {
     const int k = (p.top_k > 0 && p.top_k < n_valid) ? p.top_k : n_valid;
     if (p.temperature <= 0.0f || k <= QH_SAMPLE_MAX_TOPK) {
+        // Full logits with a workspace: the groups' maxima over the whole GPU first, so that the one workgroup reads
+        // those and about k groups instead of every logit twice and a sort of its threads' maxima (151,936 logits,
+        // top-k 20: 69 -> 18 us). Too few groups for the bound, or few logits: the one workgroup alone.
+        const int groups = (n_valid + kGroup - 1) / kGroup;
+        uint64_t* gmax = nullptr;
+        if (!rows && ws && n_valid >= 8192 && (p.temperature <= 0.0f || groups >= 2 * k)) {
+            gmax = static_cast<uint64_t*>(ws);
+            qh_launch(sample_groups_kernel, dim3((unsigned)((groups + 3) / 4)), dim3(kGroupThreads), 0, s, logits,
+                      n_valid, hist, p.repeat_penalty, gmax);
+        }
         qh_launch(sample_kernel, dim3(1), dim3(kThreads), sample_lds_bytes(n_valid), s, logits, n_valid, rows, hs,
-                  hist, p, state, out_id);
+                  hist, p, state, out_id, gmax, groups);
         return hipGetLastError();
     }
     if (!ws) return hipErrorInvalidValue;
