@@ -1064,8 +1064,17 @@ MmPlan matmul_plan(int rows, int cols, int n) {
     // down).
     const long row_tiles = (rows + 63) / 64;
     const long tiles32 = row_tiles * ((n + 31) / 32), tiles16 = row_tiles * ((n + 15) / 16);
-    if (n >= 128 && tiles32 >= 192)
-        return cols >= 2048 ? MmPlan{false, 1, 8, false, 0, true, 16, 32} : MmPlan{false, 1, 4, false, 0, true, 4, 32};
+    if (n >= 128 && tiles32 >= 192) {
+        // Long rows: eight waves with 16-block chunks keep a CU busy with one workgroup, which is all that up to one
+        // tile per CU gives it (1536x8960 at M = 300: 39.0 us, 44.0 and 52.3 for the two below). With more tiles than
+        // CUs, smaller chunks let several workgroups share a CU: four waves with 8-block chunks up to two tiles per CU
+        // (Q4_0 896x4864 at M = 1024: 37.3 us, 45.2 with eight waves, 39.3 with 4-block chunks; 1536x8960 at 512:
+        // 62.9, 73.6, 66.9), 4-block chunks beyond (4096x14336 at 300: 138.6, 165.9 with eight waves, 151.1 with 8-block
+        // chunks; Q8_0 4096x4096 at 700: 74.8, 106.9, 87.5), as on short rows.
+        const long cus = device_cus();
+        if (cols >= 2048 && tiles32 <= cus) return MmPlan{false, 1, 8, false, 0, true, 16, 32};
+        return MmPlan{false, 1, 4, false, 0, true, cols >= 2048 && tiles32 <= 2 * cus ? 8 : 4, 32};
+    }
     if (n >= 128 && cols >= 2048 && tiles16 >= 192) return MmPlan{false, 1, 4, false, 0, true, 8, 16};
     return MmPlan{false, 1, 4, true};
 }
