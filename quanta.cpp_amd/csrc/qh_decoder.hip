@@ -1658,10 +1658,22 @@ __global__ __launch_bounds__(1024) void attention_decode_kernel(
     QH_STAMP(6);
 
     // out_i = sum_j a_j * v_ji, one FMA per position in order (model.cpp:131-135): lane i of wave 0 per dimension,
-    // the weights as scalar operands (as in attention_kernel); the other waves warm the weight row's lines.
+    // the weights as scalar operands (as in attention_kernel); the other waves warm the weight row's lines and load the
+    // next stage's cache blocks into registers while the chain runs, so that only LDS stores stand between two stages
+    // (position 3,500: 37.3 -> 31.7 us a layer).
+    constexpr int kLoaders = NT - HD, kPre = (kVBlk * HD + kLoaders - 1) / kLoaders;
+    v4u nxt[kPre];
     float acc = 0.0f;
     for (int s0 = 0;;) {
         const int se = min(nrows, s0 + kVRows);
+        if (tid >= HD && se < nrows) {  // uniform per wave; pos >= 1 here (a second stage)
+            const int nb8 = (min(nrows, se + kVRows) - se + 7) / 8, lastc = (pos - 1) / 8;
+#pragma unroll
+            for (int u = 0; u < kPre; ++u) {  // units past the stage repeat its last (never stored)
+                const int c = min(tid - HD + kLoaders * u, nb8 * HD - 1);
+                nxt[u] = ld4(vc4 + vchunk(min(se / 8 + c / HD, lastc), c % HD));
+            }
+        }
         if (tid < HD) {
             const_v16f_ptr wp = (const_v16f_ptr)(arow + s0);  // s0 is a multiple of 32: 64-byte aligned
             auto ldv = [&](uint4(&vv)[4], int jr) {  // rows s0 + jr .. + 31 (jr % 32 == 0)
@@ -1731,9 +1743,12 @@ __global__ __launch_bounds__(1024) void attention_decode_kernel(
         __syncthreads();  // the stage is consumed; load rows [s0, min(nrows, s0 + kVRows)) (s0 % 8 == 0)
         const int sn = min(nrows, s0 + kVRows);
         const int nb8 = (sn - s0 + 7) / 8;
-        for (int c = tid; c < nb8 * HD; c += NT) {  // whole cache blocks; the token's row is written after
-            const int blk = s0 / 8 + c / HD, d = c % HD;
-            vst[c] = blk * 8 < pos ? vc4[vchunk(blk, d)] : make_uint4(0u, 0u, 0u, 0u);
+        if (tid >= HD) {
+#pragma unroll
+            for (int u = 0; u < kPre; ++u) {  // whole cache blocks; the token's row is written after
+                const int c = tid - HD + kLoaders * u;
+                if (c < nb8 * HD) *reinterpret_cast<v4u*>(&vst[c]) = nxt[u];
+            }
         }
         __syncthreads();
         if (pos >= s0 && pos < sn && tid < HD) vst16[(((pos - s0) >> 3) * HD + tid) * 8 + (pos & 7)] = vloc[tid];
