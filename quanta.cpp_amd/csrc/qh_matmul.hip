@@ -1059,7 +1059,7 @@ MmPlan matmul_plan(int rows, int cols, int n) {
     // 8.4 against 11.9 and 13.3) and eight waves with 16-block chunks on longer rows (Q4_0 896x4864 at M = 512: 22.4,
     // against 23.0 with 8-block chunks, 24.4 with four waves, 25.4 with 16-token workgroups). Long rows with too few
     // 32-token tiles take 16-token workgroups when they make about 192 (896x4864 at M = 256: 19.4 against 24.7
-    // staged). Everywhere else (32 and 64 tokens, few row tiles) the LDS-staged kernel wins, also over the
+    // staged). Everywhere else (few tiles) the LDS-staged kernel wins, also over the
     // register-chain kernel; it measured 4-12% under the LDS and register kernels at 32 tokens (q/k/v, o, gate/up,
     // down).
     const long row_tiles = (rows + 63) / 64;
@@ -1076,6 +1076,14 @@ MmPlan matmul_plan(int rows, int cols, int n) {
         return MmPlan{false, 1, 4, false, 0, true, cols >= 2048 && tiles32 <= 2 * cus ? 8 : 4, 32};
     }
     if (n >= 128 && cols >= 2048 && tiles16 >= 192) return MmPlan{false, 1, 4, false, 0, true, 8, 16};
+    // Below 128 tokens: 16-token tiles once there are about 192 (Q4_0 4864x896 at 77 tokens 7.6 us, 9.6 staged; 8960x1536 at
+    // 40 10.3 and 17.6; 16384x1024 at 20 8.0 and 11.8; Q8_0 12000x2048 at 64 18.6 and 36.7; fewer tiles: 4096x14336 at 20,
+    // 128 of them, 49.4 and 35.6), on long rows the eight waves where they make that many 32-token tiles, at most one per
+    // CU (4096x14336 at 100 tokens 59.0 us, 73.7 with 16-token tiles, 113.0 staged).
+    if (n < 128 && tiles16 >= 192) {
+        if (cols >= 2048 && tiles32 >= 192 && tiles32 <= device_cus()) return MmPlan{false, 1, 8, false, 0, true, 16, 32};
+        return MmPlan{false, 1, 4, false, 0, true, 8, 16};
+    }
     return MmPlan{false, 1, 4, true};
 }
 
