@@ -8,7 +8,9 @@
 //  3. top-k (sampler.cpp:39-50): the k-th largest key of any k candidates bounds the k-th largest overall from below,
 //     so each wave ranks 64 candidates (the first 64 rows of the shortlist head's list are its seeds, the best coarse
 //     scores, which makes the bound tight) and only keys at or above the best bound enter an LDS pool, which a
-//     bitonic network sorts; a pool that overflows falls back to k rounds of a block maximum below the previous key;
+//     bitonic network sorts; a pool that overflows falls back to k rounds of a block maximum below the previous key.
+//     Full logits with a workspace: the largest key of each group of ids first, over the whole GPU
+//     (sample_groups_kernel); the k-th largest of those is the bound, and only the groups that reach it are read;
 //  4. softmax with temperature, min-p, top-p and the draw (sampler.cpp:52-84): the exponentials and divisions run one
 //     per thread, the sums and the draw serially in the reference's order; glibc-identical expf; xorshift64* state in
 //     device memory.
@@ -51,44 +53,58 @@ __device__ uint64_t block_max_u64(uint64_t v, uint64_t* red) {
 
 }  // namespace
 
-// The largest key of each group of kGroup ids (every id below n_valid a candidate), 4 groups to a workgroup.
-constexpr int kGroup = 256, kGroupThreads = 256;
+// The largest key of each group of kGroup ids (every id below n_valid a candidate), a wave to a group, 4 to a workgroup.
+// A group is 16 runs of kRun consecutive ids, run r of group g being ids (r * n_groups + g) * kRun ..: a workgroup's
+// runs of one r are 64 consecutive ids, and neighbouring large logits (sorted ones, a plateau) fall into as many groups
+// as they have runs, so that the k-th largest group maximum leaves about kRun * k of them, where groups of 256
+// consecutive ids left 256 * k: past the pool's 4,096 for k above 16 (sorted logits, 151,936 of them, top-k 20: 670 us,
+// 72 in one workgroup alone, 28 now). Runs of 32 overflow it above k = 128 and read no faster.
+constexpr int kGroup = 256, kRun = 16, kGroupThreads = 256;
 __global__ __launch_bounds__(kGroupThreads) void sample_groups_kernel(const float* __restrict__ logits, int n_valid,
-                                                                      HeadMust hist, float penalty,
-                                                                      uint64_t* __restrict__ gmax) {
-    constexpr int kIds = kGroup * kGroupThreads / 64;
-    __shared__ uint32_t seen[kIds / 32];
-    const int tid = (int)threadIdx.x, first = (int)blockIdx.x * kIds;
-    float l[kGroup / 64];
-    const int id0 = first + (tid >> 6) * kGroup + (tid & 63);
+                                                                      int n_groups, uint32_t magic, HeadMust hist,
+                                                                      float penalty, uint64_t* __restrict__ gmax) {
+    constexpr int kWgGroups = kGroupThreads / 64, kPer = kGroup / 64;
+    // run / n_groups = run * magic >> 32: exact for every run (run * n_groups < 2^32), magic = 2^32 / n_groups rounded up
+    __shared__ uint32_t seen[kWgGroups * kGroup / 32];  // bit kGroup w + i: place i of wave w's group is in the history
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6, g0 = (int)blockIdx.x * kWgGroups, g = g0 + wave;
+    float l[kPer];
+    int id[kPer];
 #pragma unroll
-    for (int j = 0; j < kGroup / 64; ++j) l[j] = logits[min(id0 + 64 * j, n_valid - 1)];
+    for (int j = 0; j < kPer; ++j) {  // place 64 j + lane of the group
+        id[j] = ((64 / kRun * j + lane / kRun) * n_groups + g) * kRun + lane % kRun;
+        l[j] = logits[min(id[j], n_valid - 1)];
+    }
     if (penalty != 1.0f) {
-        if (tid < kIds / 32) seen[tid] = 0u;
+        if (tid < kWgGroups * kGroup / 32) seen[tid] = 0u;
         __syncthreads();
         const int32_t* h;
         int nh;
         must_span(hist, h, nh);
         for (int i = tid; i < nh; i += kGroupThreads) {
-            const int at = h[i] - first;
-            if (at >= 0 && at < kIds) atomicOr(&seen[at >> 5], 1u << (at & 31));
+            const int v = h[i];
+            if (v < 0 || v >= n_valid) continue;
+            const int run = v / kRun, r = (int)__umulhi((uint32_t)run, magic), at = run - r * n_groups - g0;
+            if (at >= 0 && at < kWgGroups) {
+                const int bit = kGroup * at + kRun * r + v % kRun;
+                atomicOr(&seen[bit >> 5], 1u << (bit & 31));
+            }
         }
         __syncthreads();
     }
     uint64_t m = 0;
 #pragma unroll
-    for (int j = 0; j < kGroup / 64; ++j) {
-        const int id = id0 + 64 * j, at = id - first;
-        if (penalty != 1.0f && ((seen[at >> 5] >> (at & 31)) & 1u)) l[j] = l[j] > 0 ? l[j] / penalty : l[j] * penalty;
-        const uint64_t key = id < n_valid ? score_key(l[j], id) : 0ull;
+    for (int j = 0; j < kPer; ++j) {
+        const int bit = kGroup * wave + 64 * j + lane;
+        if (penalty != 1.0f && ((seen[bit >> 5] >> (bit & 31)) & 1u)) l[j] = l[j] > 0 ? l[j] / penalty : l[j] * penalty;
+        const uint64_t key = id[j] < n_valid ? score_key(l[j], id[j]) : 0ull;
         m = key > m ? key : m;
     }
     m = wave_max_u64(m);
-    const int g = (int)blockIdx.x * (kGroupThreads / 64) + (tid >> 6);
-    if ((tid & 63) == 0 && g * kGroup < n_valid) gmax[g] = m;
+    if (lane == 0 && g < n_groups) gmax[g] = m;
 }
 
-// gmax: the groups' largest keys (n_groups of them, rows null), or null.
+// GROUPS: gmax holds the groups' largest keys (n_groups of them, at most kThreads; rows null).
+template <bool GROUPS>
 __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restrict__ logits, int n_valid,
                                                           const int32_t* __restrict__ rows,
                                                           const qh_head_stats* __restrict__ hs, HeadMust hist,
@@ -98,7 +114,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
     extern __shared__ uint32_t seen[];  // [ceil(n_valid / 32)]: history ids, when the penalty is on
     __shared__ uint64_t pool[kPool];
     __shared__ int n_list;
-    __shared__ uint32_t ghi;
+    __shared__ uint64_t gthr;
     __shared__ uint64_t red[kWaves];
     __shared__ uint64_t wbound[kWaves];
     __shared__ uint32_t survivors[2 * QH_SAMPLE_MAX_TOPK];
@@ -135,7 +151,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
 
     if (p.temperature <= 0.0f) {  // first maximum (sampler.cpp:35-37)
         uint64_t m = 0;
-        if (gmax) {
+        if constexpr (GROUPS) {
             if (tid < n_groups) m = gmax[tid];
         } else {
             for (int i = tid; i < n; i += kThreads) {
@@ -155,34 +171,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
     // so for k <= 64 the first 64 entries already hold k candidates: each wave's k-th largest of its 64 bounds it.
     // Past 1024 candidates otherwise: the k-th largest of the threads' own maxima (k distinct candidates are at or
     // above it).
-    int nc = n;  // candidates to filter: all, or those of the listed groups
-    if (gmax) {
-        // The k-th largest group maximum bounds the k-th largest key from below, and only groups whose maximum reaches
-        // it hold larger ones: wave 0 finds the largest score bits T that at least k maxima reach, bit by bit.
-        const uint64_t mine = tid < n_groups ? gmax[tid] : 0ull;
-        pool[tid] = mine;
-        if (tid == 0) pool_n = n_list = 0;
-        __syncthreads();
-        if (wave == 0) {
-            uint32_t h[kWaves];
-#pragma unroll
-            for (int w = 0; w < kWaves; ++w) h[w] = (uint32_t)(pool[64 * w + lane] >> 32);
-            uint32_t t = 0u;
-            for (int bit = 31; bit >= 0; --bit) {
-                const uint32_t c = t | (1u << bit);
-                int at_least = 0;
-#pragma unroll
-                for (int w = 0; w < kWaves; ++w) at_least += (int)__popcll(__ballot(h[w] >= c));
-                t = at_least >= k ? c : t;
-            }
-            if (lane == 0) ghi = t;
-        }
-        __syncthreads();
-        thr = (uint64_t)ghi << 32;
-        if (mine != 0 && mine >= thr) glist[atomicAdd(&n_list, 1)] = (uint16_t)tid;
-        __syncthreads();
-        nc = n_list * kGroup;
-    } else if (n > kThreads && (!rows || k > 64)) {
+    auto strided_bound = [&]() {
         uint64_t m = 0;
 #pragma unroll 8
         for (int i = tid; i < n; i += kThreads) {
@@ -195,6 +184,84 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
         bitonic_sort_desc_u64<kThreads>(pool, kThreads);
         thr = pool[k - 1];
         __syncthreads();  // pool is refilled below
+    };
+    auto filter = [&]() {        // the candidates at or above the bound, into the pool
+        thr = thr ? thr : 1ull;  // no bound: every real key (keys are nonzero)
+#pragma unroll 8
+        for (int i = tid; i < n; i += kThreads) {
+            const uint64_t key = key_of(i);
+            if (key >= thr) {
+                const int at = atomicAdd(&pool_n, 1);
+                if (at < kPool) pool[at] = key;
+            }
+        }
+        __syncthreads();
+    };
+    if constexpr (GROUPS) {
+        // The k-th largest group maximum bounds the k-th largest key from below, and only groups whose maximum reaches
+        // it hold larger ones. Wave 0 finds it bit by bit: the largest score bits T that at least k maxima reach and,
+        // where many more than k do (equal logits, -inf of a mask), how small the ids with score T may be kept.
+        const uint64_t mine = tid < n_groups ? gmax[tid] : 0ull;
+        pool[tid] = mine;
+        if (tid == 0) pool_n = n_list = 0;
+        __syncthreads();
+        auto bound = [&](auto words) {  // over the first 64 * words places, the groups' among them
+            constexpr int W = decltype(words)::value;
+            uint32_t h[W];
+#pragma unroll
+            for (int w = 0; w < W; ++w) h[w] = (uint32_t)(pool[64 * w + lane] >> 32);
+            auto reach = [&](uint32_t c) {
+                int at_least = 0;
+#pragma unroll
+                for (int w = 0; w < W; ++w) at_least += (int)__popcll(__ballot(h[w] >= c));
+                return at_least;
+            };
+            uint32_t t = 0u, low = 0u;
+            for (int bit = 31; bit >= 0; --bit) {
+                const uint32_t c = t | (1u << bit);
+                t = reach(c) >= k ? c : t;
+            }
+            if (reach(t) > k + 8) {  // uniform; within 8 of k the ties add few candidates
+                const int need = k - (t == 0xffffffffu ? 0 : reach(t + 1u));  // of the maxima with score T, lowest ids
+#pragma unroll
+                for (int w = 0; w < W; ++w) h[w] = h[w] == t ? (uint32_t)pool[64 * w + lane] : 0u;
+                for (int bit = 31; bit >= 4; --bit) {  // the low word is ~id, the bits above the ids' all ones
+                    const uint32_t c = low | (1u << bit);
+                    low = ((uint32_t)(n_valid - 1) >> bit) == 0u || reach(c) >= need ? c : low;
+                }
+            }
+            if (lane == 0) gthr = (uint64_t)t << 32 | low;
+        };
+        if (wave == 0) {
+            if (n_groups <= 256)  // uniform
+                bound(std::integral_constant<int, 4>{});
+            else
+                bound(std::integral_constant<int, kWaves>{});
+        }
+        __syncthreads();
+        thr = gthr;
+        if (mine != 0 && mine >= thr) glist[atomicAdd(&n_list, 1)] = (uint16_t)tid;
+        __syncthreads();
+        thr = thr ? thr : 1ull;
+        const int nc = n_list * kGroup;
+#pragma unroll 8
+        for (int c = tid; c < nc; c += kThreads) {
+            const int in = c % kGroup, i = (in / kRun * n_groups + glist[c / kGroup]) * kRun + in % kRun;
+            const uint64_t key = i < n ? key_of(i) : 0ull;
+            if (key >= thr) {
+                const int at = atomicAdd(&pool_n, 1);
+                if (at < kPool) pool[at] = key;
+            }
+        }
+        __syncthreads();
+        if (pool_n > kPool) {  // uniform; logits crowded into few groups: the bound over strided candidates instead
+            __syncthreads();
+            strided_bound();
+            filter();
+        }
+    } else if (n > kThreads && (!rows || k > 64)) {
+        strided_bound();
+        filter();
     } else {  // the k-th largest of each wave's 64 candidates (when k <= 64)
         const int i = wave * 64 + lane;
         const uint64_t a = i < n ? key_of(i) : 0ull;
@@ -213,18 +280,8 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
         thr = wbound[0];
 #pragma unroll
         for (int w = 1; w < kWaves; ++w) thr = wbound[w] > thr ? wbound[w] : thr;
+        filter();
     }
-    thr = thr ? thr : 1ull;  // no bound: every real key (keys are nonzero)
-#pragma unroll 8
-    for (int c = tid; c < nc; c += kThreads) {
-        const int i = gmax ? glist[c / kGroup] * kGroup + c % kGroup : c;
-        const uint64_t key = i < n ? key_of(i) : 0ull;
-        if (key >= thr) {
-            const int at = atomicAdd(&pool_n, 1);
-            if (at < kPool) pool[at] = key;
-        }
-    }
-    __syncthreads();
     const int count = pool_n;
     if (count == 0) {  // uniform; no candidate (an empty row list)
         if (tid == 0) *out_id = 0;
@@ -587,16 +644,21 @@ hipError_t launch_sample(const float* logits, int n_valid, const int32_t* rows, 
     if (p.temperature <= 0.0f || k <= QH_SAMPLE_MAX_TOPK) {
         // Full logits with a workspace: the groups' maxima over the whole GPU first, so that the one workgroup reads
         // those and about k groups instead of every logit twice and a sort of its threads' maxima (151,936 logits,
-        // top-k 20: 69 -> 18 us). Too few groups for the bound, or few logits: the one workgroup alone.
+        // top-k 20: 72 -> 20 us). Too few groups for the bound, or few logits (greedy over 8,192: 6.9 us in two
+        // launches, 6.2 in one; 33,000: 6.8 and 11.2): the one workgroup alone.
         const int groups = (n_valid + kGroup - 1) / kGroup;
-        uint64_t* gmax = nullptr;
-        if (!rows && ws && n_valid >= 8192 && (p.temperature <= 0.0f || groups >= 2 * k)) {
-            gmax = static_cast<uint64_t*>(ws);
+        const bool greedy = p.temperature <= 0.0f;
+        const size_t lds = sample_lds_bytes(n_valid);
+        if (!rows && ws && (greedy ? n_valid >= 16384 : n_valid >= 8192 && groups >= 2 * k)) {
+            uint64_t* gmax = static_cast<uint64_t*>(ws);
             qh_launch(sample_groups_kernel, dim3((unsigned)((groups + 3) / 4)), dim3(kGroupThreads), 0, s, logits,
-                      n_valid, hist, p.repeat_penalty, gmax);
+                      n_valid, groups, 0xffffffffu / (uint32_t)groups + 1u, hist, p.repeat_penalty, gmax);
+            qh_launch((sample_kernel<true>), dim3(1), dim3(kThreads), lds, s, logits, n_valid, rows, hs, hist, p, state,
+                      out_id, gmax, groups);
+        } else {
+            qh_launch((sample_kernel<false>), dim3(1), dim3(kThreads), lds, s, logits, n_valid, rows, hs, hist, p, state,
+                      out_id, (const uint64_t*)nullptr, 0);
         }
-        qh_launch(sample_kernel, dim3(1), dim3(kThreads), sample_lds_bytes(n_valid), s, logits, n_valid, rows, hs,
-                  hist, p, state, out_id, gmax, groups);
         return hipGetLastError();
     }
     if (!ws) return hipErrorInvalidValue;

@@ -32,3 +32,52 @@ def test_group_filter_equals_single_workgroup(qh, gpu, n, kind):
             ids = [int(qh.sample(logits, p, state, history=h, ws=w)[0]) for _ in range(3)]
             got.append((ids, int(state[0])))
         assert got[0] == got[1], (k, temp, pen)
+
+
+def _crowded(kind, n, g):
+    """Logits whose largest fall together along the ids: sorted, masked to a few ids, equal, a slow wave, or all of
+    20 whole groups (16 runs of 16 ids, a group's runs ceil(n / 256) runs apart), each above the one before."""
+    if kind == "sorted":
+        return np.sort(g.standard_normal(n) * 3)[::-1].astype(np.float32)
+    if kind == "masked":
+        x = np.full(n, -np.inf, np.float32)
+        x[g.integers(0, n, 9)] = g.standard_normal(9)
+        return x
+    if kind == "equal":
+        return np.zeros(n, np.float32)
+    if kind == "wave":
+        return (3 * np.sin(np.arange(n) * (2 * np.pi / 3000))).astype(np.float32)
+    group = np.arange(n) // 16 % ((n + 255) // 256)
+    return np.where(group < 20, 10 + group, 0).astype(np.float32) + g.random(n).astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", ["sorted", "masked", "equal", "wave", "levels"])
+@pytest.mark.parametrize("n", [33001, 151936, 262144])
+def test_crowded_logits_equal_single_workgroup_and_take_no_longer(qh, gpu, n, kind):
+    """The same draw, and in no more time than one workgroup alone takes, give or take the timer (measured 0.2 to 1.3 of
+    it; a pool that overflows into k passes over the logits takes 5 to 100 times as long)."""
+    import torch
+    g = np.random.default_rng(n)
+    x = _crowded(kind, n, g)
+    logits = torch.from_numpy(np.ascontiguousarray(x)).to(gpu)
+    ws = qh.sample_workspace(n)
+    hist = torch.from_numpy(g.integers(0, n, 300).astype(np.int32)).to(gpu)
+    for k in (17, 20, 64, 128, 256):
+        got, us = [], []
+        for w in (None, ws):
+            state = torch.full((1,), qh.sampler_state(5), dtype=torch.int64, device=gpu)
+            p = qh.sampler_params(top_k=k, top_p=0.95)
+            ids = [int(qh.sample(logits, p, state, history=hist, ws=w)[0]) for _ in range(3)]
+            got.append((ids, int(state[0])))
+            times = []
+            for _ in range(7):
+                a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                a.record()
+                for _ in range(8):
+                    qh.sample(logits, p, state, history=hist, ws=w)
+                b.record()
+                b.synchronize()
+                times.append(a.elapsed_time(b))
+            us.append(sorted(times)[3] * 125)
+        assert got[0] == got[1], k
+        assert us[1] <= 2.5 * us[0], (k, us)
