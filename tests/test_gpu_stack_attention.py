@@ -75,3 +75,22 @@ def test_stack_attention_infinite_values(qh, gpu, turns):
     scales[:] = (scales.astype(np.float32) * 3e5).astype(np.float16)  # |v| reaches 65,504 at a few positions
     tens["model.layers.0.self_attn.v_proj.weight"] = qnt.TensorRec(rec.dtype, rec.rows, rec.cols, data)
     _compare(qh, hp, tens, 1600, 512, turns)
+
+
+@pytest.mark.parametrize("n_heads,n_kv,head_dim,ctx,stack,turns", [
+    # up to 1,024 rows a workgroup takes four tokens of a head (up to 819 workgroups at position 0, 512 later on a
+    # 256-CU GPU) or 16 pairs; past them a head and token (up to 512, or 1,024 on few rows) or pair groups
+    (14, 2, 64, 1400, 256, (231, 145, 146, 236, 33, 36, 37, 73, 74, 200)),
+    (4, 1, 64, 1800, 1024, (819, 64, 128, 129, 256, 257)),
+    (6, 6, 64, 1450, 512, (35, 340, 420, 85, 200, 170, 171)),
+    # head_dim 128: a head and token for one round of workgroups, or two past a mean of 200 rows, to 1,024 rows; one
+    # round to 2,700
+    (4, 2, 128, 1300, 256, (64, 65, 128, 129, 256, 128, 129, 63, 64, 65)),
+    (2, 1, 128, 2900, 1024, (2600, 64, 64, 129)),
+])
+def test_small_stacks_equal_chunks(qh, gpu, n_heads, n_kv, head_dim, ctx, stack, turns):
+    """Turns on both sides of the sizes where the stack's attention changes kernel by its number of workgroups."""
+    qnt = qnt_module()
+    hp = qnt.HParams(vocab_size=512, dim=n_heads * head_dim, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv,
+                     head_dim=head_dim, ffn_dim=512)
+    _compare(qh, hp, qnt.synthetic_q4mix(83 + n_heads, hp, shortlist=False), ctx, stack, turns, seed=5)
