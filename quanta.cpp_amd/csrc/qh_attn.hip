@@ -652,16 +652,20 @@ __global__ __launch_bounds__(256) void attn_short_kernel(AttnStack a, int ng16) 
 
 // Workspace floats per (pair group, KV head) whose last token has `rows` rows: the scores, the score waves' maxima (at
 // least 32 positions each) and the inverse sums.
-constexpr size_t kWsPad = 4 * kValTile * 256;  // rows that attn_values_kernel loads past a group's and never uses
+constexpr size_t kWsPad = 4 * kValTile * 256;  // bytes: four tiles of rows that attn_values_kernel may load past a group's
 size_t group_floats(int rs) { return 64 * ((size_t)rs + rs / 32 + 1); }
 int row_stride(int rows) { return (rows + kRowPad - 1) / kRowPad * kRowPad; }
 
 }  // namespace
 
-// Bytes for `tokens` at the end of the context, at most kAttnWsBytes unless one token's pairs need more.
-size_t attn_stack_ws_bytes(int n_heads, int n_kv, int ctx, int tokens) {
+// Bytes for `tokens` at the end of the context, at most kAttnWsBytes unless one token's pairs need more, which is the
+// least that works (*least); 0 for a context whose every stack one launch takes.
+size_t attn_stack_ws_bytes(int n_heads, int n_kv, int ctx, int tokens, size_t* least_bytes) {
+    *least_bytes = 0;
+    if (ctx <= kShortRows) return 0;
     const size_t G = (size_t)(n_heads / n_kv), groups = (tokens * G + 63) / 64, least = (G + 63) / 64;
     const size_t per = (size_t)n_kv * group_floats(row_stride(ctx)) * 4, fit = kAttnWsBytes / per;
+    *least_bytes = per * least + kWsPad;
     return per * (groups < fit ? groups : fit > least ? fit : least) + kWsPad;
 }
 

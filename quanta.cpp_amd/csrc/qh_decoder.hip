@@ -2469,10 +2469,18 @@ hipError_t alloc_stack(Decoder* d, int c) {
         A((void**)&d->fb, sizeof(float) * c * wide);
     }
     A((void**)&d->subpos, sizeof(int) * (kMaxStack / kChunk));
-    if (c > kChunk && !d->kv32) {
-        const size_t b = attn_stack_ws_bytes(hp.n_heads, hp.n_kv_heads, hp.ctx_len, c);
-        A((void**)&d->aws, b);
-        if (e == hipSuccess) d->aws_bytes = b;
+    // the stack attention's scores, where it runs: any size from the least works, so less is taken where the rest of
+    // the memory is in use
+    size_t least = 0, b = c > kChunk && !d->kv32 && d->fuse
+                              ? attn_stack_ws_bytes(hp.n_heads, hp.n_kv_heads, hp.ctx_len, c, &least) : 0;
+    for (; b && e == hipSuccess; b = b / 2 < least ? least : b / 2) {
+        e = dalloc(d, (void**)&d->aws, b);
+        if (e == hipSuccess) {
+            d->aws_bytes = b;
+            break;
+        }
+        (void)hipGetLastError();
+        if (e == hipErrorOutOfMemory && b > least) e = hipSuccess;
     }
     return e;
 }

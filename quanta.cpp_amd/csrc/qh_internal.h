@@ -185,10 +185,10 @@ struct AttnStack {
     int8_t* oq;
     float *od, *of;
     int rs;              // workspace rows per pair group
-    float *s, *pm, *inv;  // scores [n_kv * groups][rs / 4][64][4], maxima, inverse sums
+    float *s, *pm, *inv;  // scores [n_kv * groups][rs / 16][4][4][16][4] (qh_attn.hip), maxima, inverse sums
 };
 constexpr size_t kAttnWsBytes = (size_t)256 << 20;
-size_t attn_stack_ws_bytes(int n_heads, int n_kv, int ctx, int tokens);
+size_t attn_stack_ws_bytes(int n_heads, int n_kv, int ctx, int tokens, size_t* least_bytes);
 hipError_t launch_attention_stack(AttnStack a, int head_dim, float* ws, size_t ws_bytes, hipStream_t s);
 
 // GPU-resident decoder (qh_decoder.hip). Tensors in qh_decoder_create order; all sizes validated by the caller.

@@ -94,3 +94,44 @@ def test_small_stacks_equal_chunks(qh, gpu, n_heads, n_kv, head_dim, ctx, stack,
     hp = qnt.HParams(vocab_size=512, dim=n_heads * head_dim, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv,
                      head_dim=head_dim, ffn_dim=512)
     _compare(qh, hp, qnt.synthetic_q4mix(83 + n_heads, hp, shortlist=False), ctx, stack, turns, seed=5)
+
+
+def _wide(qnt):
+    hp = qnt.HParams(vocab_size=512, dim=1024, n_layers=1, n_heads=16, n_kv_heads=2, head_dim=64, ffn_dim=512)
+    return hp, qnt.synthetic_q4mix(17, hp, shortlist=False)
+
+
+def test_stack_takes_no_score_workspace_for_a_short_context(qh, gpu):
+    """A context of up to 1,024 rows never goes through the score workspace (69 MB for this model's 1,024-token stack):
+    setting the stack takes its work buffers (about 20 MB) and no more."""
+    import torch
+    qnt = qnt_module()
+    hp, tens = _wide(qnt)
+    dec = qh.Decoder(hp, tens, ctx_len=1024)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    dec.set_prefill_stack(1024)
+    taken = free - torch.cuda.mem_get_info()[0]
+    dec.close()
+    assert taken < 48 << 20, taken
+
+
+def test_stack_with_a_smaller_score_workspace(qh, gpu):
+    """Where the score workspace cannot be allocated whole the stack is still set, with half of it (here its allocation,
+    the thirteenth, is made to fail), and its attention takes the stack in more passes with the same results."""
+    qnt = qnt_module()
+    hp, tens = _wide(qnt)
+    ids = np.random.default_rng(9).integers(0, hp.vocab_size, 1800).astype(np.int32)
+    got = []
+    for after in (-1, 12):
+        dec = qh.Decoder(hp, tens, ctx_len=1900)
+        try:
+            qh.lib().qh_fault_alloc(after)
+            dec.set_prefill_stack(1024)
+        finally:
+            qh.lib().qh_fault_alloc(-1)
+        dec.prefill(ids, 0, top_k=0)
+        got.append((dec.hidden(), dec.kv(0, len(ids))))
+        dec.close()
+    assert _equal(got[0][0], got[1][0])
+    assert all(_equal(a, b) for a, b in zip(got[0][1], got[1][1]))
