@@ -2372,8 +2372,8 @@ struct Decoder {
     size_t aws_bytes = 0;
     int32_t* tokens = nullptr;  // [kChunk] prefill input / [0] decode input
     // Prefill stack: the tokens whose norms and matmuls share one launch (kChunk, the reference's Model::kBatch, by
-    // default; larger stacks run the matmul tile kernels at M up to kMaxStack). Attention runs each stack as 32-token
-    // sub-chunks in order, the sub-chunk i starting at subpos[i].
+    // default; larger stacks run the matmul tile kernels at M up to kMaxStack). Over an f32 cache, or without the fused
+    // kernels, attention runs each stack as 32-token sub-chunks in order, the sub-chunk i starting at subpos[i].
     int stack = kChunk;
     int* subpos = nullptr;
     int stack_end = 0;  // the current prefill stack's end position (host-side, for the attention plan)
@@ -2443,6 +2443,9 @@ void dfree(Decoder* d, void* p) {
     (void)hipFree(p);
 }
 
+// Whether a prefill stack's tokens go through attention together (attention_stack), not as 32-token sub-chunks.
+bool stack_attention(const Decoder* d) { return d->fuse && !d->kv32; }
+
 // The work buffers of a prefill stack of c tokens: the residual stream, projections, MLP rows, int8 activations and
 // their scales, the f32 copies for unquantized matrices and the attention sub-chunks' positions. On failure the ones
 // allocated stay listed (the caller frees them).
@@ -2471,7 +2474,7 @@ hipError_t alloc_stack(Decoder* d, int c) {
     A((void**)&d->subpos, sizeof(int) * (kMaxStack / kChunk));
     // the stack attention's scores, where it runs: any size from the least works, so less is taken where the rest of
     // the memory is in use
-    size_t least = 0, b = c > kChunk && !d->kv32 && d->fuse
+    size_t least = 0, b = c > kChunk && stack_attention(d)
                               ? attn_stack_ws_bytes(hp.n_heads, hp.n_kv_heads, hp.ctx_len, c, &least) : 0;
     for (; b && e == hipSuccess; b = b / 2 < least ? least : b / 2) {
         e = dalloc(d, (void**)&d->aws, b);
@@ -2802,8 +2805,8 @@ hipError_t attention_stack(Decoder* d, int l, int n, hipStream_t s) {
 
 hipError_t attention(Decoder* d, int l, int n, hipStream_t s) {
     const qh_model_desc& hp = d->hp;
-    if (n > kChunk && !d->kv32 && d->fuse) return attention_stack(d, l, n, s);
-    if (n > kChunk) {  // a prefill stack: its 32-token sub-chunks in order (each reads the rows the ones before wrote)
+    if (n > kChunk && stack_attention(d)) return attention_stack(d, l, n, s);
+    if (n > kChunk) {  // a prefill stack without it: its 32-token sub-chunks in order (each reads the rows the ones before wrote)
         for (int i = 0; i * kChunk < n; ++i)
             QH_TRY(attention_chunk(d, l, min(kChunk, n - i * kChunk), i * kChunk, d->subpos + i, s));
         return hipSuccess;
@@ -3130,7 +3133,7 @@ hipError_t decoder_prefill(Decoder* d, const int32_t* tokens, int n, int pos0, i
     int last = 0;
     for (int c0 = 0; c0 < n; c0 += d->stack) {
         const int m = n - c0 < d->stack ? n - c0 : d->stack;
-        if (m > kChunk) {
+        if (m > kChunk && !stack_attention(d)) {
             qh_launch(set_subpos_kernel, dim3(1), dim3(kMaxStack / kChunk), 0, s, d->subpos, pos0 + c0,
                       (m + kChunk - 1) / kChunk);
             QH_TRY(hipGetLastError());
