@@ -8,7 +8,10 @@
 // stage the next, 256 columns at a time, coalesced and widened; wave 1 also brings the next tile's activation lines
 // into the scalar cache. Against 64 rows to a workgroup with the activation from LDS: F16 896x4864 53 -> 23 us,
 // 200x14336 154 -> 62 us, F32 9000x8192 113 -> 79 us, F16 4864x896 11 -> 7 us (the call). With many rows the
-// memory bounds it, not the chain, and a workgroup takes 64 rows by 64 columns (gemv_rows).
+// memory bounds it, not the chain, and a workgroup takes 64 rows by 64 columns, with or without loading waves
+// (gemv_form). The arguments of a launch of one matrix are plain values, which are in registers when a wave starts; out
+// of the three matrices' struct they cost every wave a read of the kernel's arguments before its first load (0.1 us a
+// round of workgroups: F16 60000x256 8.0 -> 7.5 us, F32 16384x128 4.3 -> 3.8).
 // Several tokens: the chains of 16 rows x 16 tokens are an f32 matrix product summed in order (v_mfma_f32_16x16x4_f32:
 // each k step one fused multiply-add, see qh_attn.hip), 32 rows x 32 tokens to a workgroup of four waves, weights and
 // activations staged in LDS in operand order, 64 columns at a time.
@@ -34,6 +37,8 @@ struct DenseSeg {
     const uint8_t* w;
     float* out;
     int ldo, r0, r1;
+    __device__ __forceinline__ DenseSeg(const uint8_t* w_, float* out_, int r0_, int r1_)
+        : w(w_), out(out_), ldo(0), r0(r0_), r1(r1_) {}
     __device__ __forceinline__ DenseSeg(const DenseSegs& g, int& t) {  // t: the launch's row tile, then the matrix's
         int s = 0;
         if (t >= g.tiles[0]) {
@@ -71,10 +76,11 @@ constexpr int kGvLoaders = 192;
 
 }  // namespace
 
-// res: out[r] = res[r] + acc (a residual stream, read and written by the same lane), or null.
-template <int DT, int kGvRows>
-__global__ __launch_bounds__(256) void gemv_dense_kernel(DenseSegs segs, int cols, const float* __restrict__ x,
-                                                         const float* res) {
+// ONE: the matrix is w0 / out0, rows [r0, r1); else segs has them. res: out[r] = res[r] + acc (a residual stream, read
+// and written by the same lane), or null.
+template <int DT, int kGvRows, bool ONE>
+__global__ __launch_bounds__(256) void gemv_dense_kernel(const uint8_t* __restrict__ w0, float* out0, const float* __restrict__ x,
+                                                         const float* res, int cols, int r0, int r1, DenseSegs segs) {
     constexpr int kGvCols = 4096 / kGvRows, kGvStride = kGvCols + 4;
     constexpr int kSize = DT == kF32 ? 4 : 2, kPer = 16 / kSize;                    // bytes per weight, weights per unit
     constexpr int kUnits = (kGvRows * kGvCols / kPer + kGvLoaders - 1) / kGvLoaders;  // units per loading thread
@@ -82,7 +88,7 @@ __global__ __launch_bounds__(256) void gemv_dense_kernel(DenseSegs segs, int col
     __shared__ __align__(16) float ws[2][kGvRows * kGvStride];
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int rt = (int)blockIdx.x;
-    const DenseSeg sg(segs, rt);
+    const DenseSeg sg = ONE ? DenseSeg(w0, out0, r0, r1) : DenseSeg(segs, rt);
     const int rbase = sg.r0 + rt * kGvRows, ntiles = (cols + kGvCols - 1) / kGvCols;
     if (wave == 0) {
         float acc = 0.0f;
@@ -193,6 +199,69 @@ __global__ __launch_bounds__(256) void gemv_dense_kernel(DenseSegs segs, int col
     }
 }
 
+// The same for short rows, or where many rows bound it: every wave loads and stages 64 rows by 64 columns (the LDS rows
+// one bank apart), the next tile's loads in flight under this one's chains, which wave 0 runs with the activation as LDS
+// broadcasts. No hand-over between waves, and a third more of them loading.
+template <int DT, bool ONE>
+__global__ __launch_bounds__(256) void gemv_dense_plain_kernel(const uint8_t* __restrict__ w0, float* out0, const float* __restrict__ x,
+                                                         const float* res, int cols, int r0, int r1, DenseSegs segs) {
+    constexpr int kRows = 64, kCols = 64, kStride = kCols + 1;
+    constexpr int kSize = DT == kF32 ? 4 : 2, kPer = 16 / kSize, kUpr = kCols / kPer;  // weights, units per row
+    constexpr int kUnits = kRows * kUpr / 256;
+    __shared__ float ws[2][kRows * kStride];
+    __shared__ __align__(16) float xs[2][kCols];
+    const int tid = (int)threadIdx.x;
+    int rt = (int)blockIdx.x;
+    const DenseSeg sg = ONE ? DenseSeg(w0, out0, r0, r1) : DenseSeg(segs, rt);
+    const int rbase = sg.r0 + rt * kRows, row = rbase + tid, ntiles = (cols + kCols - 1) / kCols;
+    uint4 w[kUnits];
+    float4 xr = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto load = [&](int c0) {  // rows past r1 and columns past cols are clamped (loaded, never used)
+#pragma unroll
+        for (int j = 0; j < kUnits; ++j) {
+            const int u = 256 * j + tid, r = min(rbase + u / kUpr, sg.r1 - 1), c = min(c0 + kPer * (u % kUpr), cols - kPer);
+            w[j] = *reinterpret_cast<const uint4*>(sg.w + ((size_t)r * cols + c) * kSize);
+        }
+        if (tid < kCols / 4) xr = *reinterpret_cast<const float4*>(x + min(c0 + 4 * tid, cols - 4));
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int j = 0; j < kUnits; ++j) {
+            const int u = 256 * j + tid;
+            float f[kPer];
+            widen<DT>(w[j], f);
+            float* d = &ws[buf][(u / kUpr) * kStride + kPer * (u % kUpr)];
+#pragma unroll
+            for (int e = 0; e < kPer; ++e) d[e] = f[e];
+        }
+        if (tid < kCols / 4) reinterpret_cast<float4*>(xs[buf])[tid] = xr;
+    };
+    const bool run = tid < kRows && row < sg.r1;
+    const float rv = res && run ? res[row] : 0.0f;
+    float acc = 0.0f;
+    load(0);
+    stage(0);
+    __syncthreads();
+    for (int t = 0; t < ntiles; ++t) {
+        const int buf = t & 1;
+        if (t + 1 < ntiles) load((t + 1) * kCols);
+        if (run) {
+            const float* wrow = &ws[buf][tid * kStride];
+            const float* xt = xs[buf];
+            if (cols - t * kCols >= kCols) {
+#pragma unroll
+                for (int c = 0; c < kCols; ++c) acc = __builtin_fmaf(wrow[c], xt[c], acc);
+            } else {  // cols % 32 == 0
+#pragma unroll
+                for (int c = 0; c < kCols / 2; ++c) acc = __builtin_fmaf(wrow[c], xt[c], acc);
+            }
+        }
+        if (t + 1 < ntiles) stage(buf ^ 1);
+        __syncthreads();
+    }
+    if (run) sg.out[row] = res ? rv + acc : acc;
+}
+
 namespace {
 constexpr int kMmTile = 32, kMmCols = 64;
 }
@@ -299,11 +368,29 @@ __global__ __launch_bounds__(256) void matmul_dense_kernel(DenseSegs segs, int c
     }
 }
 
-// Rows per workgroup of the one-token launch: 64 where a launch has so many workgroups of 16 that their starts and loads,
-// not their chains, bound it (F16 30000x1024 18.5 us with 16, 14.9 with 64; F32 16384x448 8.3 and 6.9; F16 151936x896 66
-// and 50), 16 below and for long rows (F16 16384x14336 100 us with 16, 192 with 64; F32 4864x896 8.4 and 10.8).
-static int gemv_rows(int rows, int cols) {
-    return rows >= 128 * device_cus() || (rows >= 32 * device_cus() && cols < 4096) ? 64 : 16;
+// The one-token launch. 64 rows per workgroup where a launch has so many workgroups of 16 that their starts and loads,
+// not their chains, bound it (F16 30000x1024 18.5 us with 16, 14.9 with 64; F32 16384x448 8.3 and 6.7; F16 151936x896 68
+// and 53), 16 below and for long rows (F16 16384x14336 100 us with 16, 192 with 64; F32 4096x896 7.0 and 8.1, 32768x8192
+// 241 and 256). The plain kernel
+//   for a tile of columns or half (F32 20000x32 2.5 us, 2.8 with loading waves; 128x64 2.1 and 2.25; F16 8192x32 2.40 and
+//     2.44, 8192x64 2.54 and 2.47),
+//   for short F32 rows by the tens of thousands (100000x128 10.9 and 12.7; 12000x128 3.6 and 3.5, 100000x256 21.5 and
+//     20.4),
+//   where two to four workgroups share a CU in one round (F32 45000x448 16.0 and 16.8, 16384x448 7.4 and 6.7, 80000x1024
+//     70 and 60; F16 60000x192 6.1 and 6.6, 60000x448 11.7 and 11.9, 32768x256 5.6 and 5.2, 80000x192 8.3 and 8.1), and
+//   for long F32 rows that workgroups of 16 would take in a round and a half, four to a CU (24000x8192 172 and 182 us,
+//     28000x8192 224 and 216).
+struct GemvForm {
+    int rows;  // per workgroup
+    bool plain;
+};
+static GemvForm gemv_form(int dtype, int rows, int cols) {
+    const long cus = device_cus();
+    const bool f32 = dtype == kF32;
+    const bool one_round = rows > 128 * cus && rows <= 256 * cus && cols <= (f32 ? 1024 : 256);
+    const bool uneven = f32 && cols >= 8192 && rows > 64 * cus && rows <= 96 * cus;
+    if (cols <= (f32 ? 64 : 32) || one_round || uneven || (f32 && rows > 64 * cus && cols <= 192)) return {64, true};
+    return {cols < 8192 && (rows >= 128 * cus || (rows >= 32 * cus && cols < 4096)) ? 64 : 16, false};
 }
 
 hipError_t launch_dense_segs(const MmOut* m, int n_mats, const float* x, int ldx, int n, const float* res, hipStream_t s) {
@@ -312,7 +399,8 @@ hipError_t launch_dense_segs(const MmOut* m, int n_mats, const float* x, int ldx
     DenseSegs sg{};
     int tiles = 0, rows = 0;
     for (int i = 0; i < n_mats; ++i) rows += m[i].r1 - m[i].r0;
-    const int tile = n > 1 ? kMmTile : gemv_rows(rows, W.cols);
+    const GemvForm form = gemv_form(W.dtype, rows, W.cols);
+    const int tile = n > 1 ? kMmTile : form.rows;
     for (int i = 0; i < n_mats; ++i) {
         if (m[i].W->dtype != W.dtype || m[i].W->cols != W.cols) return hipErrorInvalidValue;
         sg.w[i] = static_cast<const uint8_t*>(m[i].W->data);
@@ -325,14 +413,30 @@ hipError_t launch_dense_segs(const MmOut* m, int n_mats, const float* x, int ldx
     }
     if (W.dtype != kF32 && W.dtype != kF16) return hipErrorInvalidValue;
     if (n == 1) {
-        if (W.dtype == kF32 && tile == 16)
-            qh_launch((gemv_dense_kernel<kF32, 16>), dim3((unsigned)tiles), dim3(256), 0, s, sg, W.cols, x, res);
-        else if (W.dtype == kF32)
-            qh_launch((gemv_dense_kernel<kF32, 64>), dim3((unsigned)tiles), dim3(256), 0, s, sg, W.cols, x, res);
-        else if (tile == 16)
-            qh_launch((gemv_dense_kernel<kF16, 16>), dim3((unsigned)tiles), dim3(256), 0, s, sg, W.cols, x, res);
+        const dim3 grid((unsigned)tiles);
+        auto launch = [&](auto dt, auto one) {
+            constexpr int DT = decltype(dt)::value;
+            constexpr bool ONE = decltype(one)::value;
+            if (form.plain)
+                qh_launch((gemv_dense_plain_kernel<DT, ONE>), grid, dim3(256), 0, s, sg.w[0], sg.out[0], x, res, W.cols,
+                          sg.r0[0], sg.r1[0], sg);
+            else if (tile == 16)
+                qh_launch((gemv_dense_kernel<DT, 16, ONE>), grid, dim3(256), 0, s, sg.w[0], sg.out[0], x, res, W.cols,
+                          sg.r0[0], sg.r1[0], sg);
+            else
+                qh_launch((gemv_dense_kernel<DT, 64, ONE>), grid, dim3(256), 0, s, sg.w[0], sg.out[0], x, res, W.cols,
+                          sg.r0[0], sg.r1[0], sg);
+        };
+        auto typed = [&](auto one) {
+            if (W.dtype == kF32)
+                launch(std::integral_constant<int, kF32>{}, one);
+            else
+                launch(std::integral_constant<int, kF16>{}, one);
+        };
+        if (n_mats == 1)
+            typed(std::true_type{});
         else
-            qh_launch((gemv_dense_kernel<kF16, 64>), dim3((unsigned)tiles), dim3(256), 0, s, sg, W.cols, x, res);
+            typed(std::false_type{});
         return hipGetLastError();
     }
     const int n_tg = (n + kMmTile - 1) / kMmTile;

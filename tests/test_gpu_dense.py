@@ -40,3 +40,26 @@ def test_dense_prompt_equals_oracle(qh, oracle, gpu, dtype, n):
     ids = np.random.default_rng(n).integers(0, hp.vocab_size, n).astype(np.int32)
     _steps_vs_oracle(oracle, orc, dec, ids, 3, shortlist=False)
     dec.close()
+
+
+@pytest.mark.parametrize("dtype", [F32, F16])
+@pytest.mark.parametrize("rows,cols", [(8191, 416), (8193, 416), (16384, 192), (16385, 192), (16385, 224), (32769, 256),
+                                       (32769, 288), (65536, 64), (65537, 64), (63, 32), (65, 64), (33, 96)])
+def test_matvec_ref_forms_equal_oracle(qh, oracle, gpu, dtype, rows, cols):
+    """Both sides of the lines between the one-token forms (16 or 64 rows to a workgroup, with or without loading
+    waves)."""
+    test_matvec_ref_tiles_equal_oracle(qh, oracle, gpu, dtype, rows, cols)
+
+
+@pytest.mark.parametrize("dtype,ffn", [(F16, 4128), (F32, 8224)])
+def test_merged_projections_in_many_rows_equal_oracle(qh, oracle, gpu, dtype, ffn):
+    """Gate and up of one token in one launch of 64 rows to a workgroup (F16: 8,256 rows, with loading waves; F32: 16,448
+    without), the second matrix beginning inside the grid."""
+    qnt = qnt_module()
+    hp = qnt.HParams(vocab_size=300, dim=64, n_layers=1, n_heads=1, n_kv_heads=1, head_dim=64, ffn_dim=ffn)
+    tens = qnt.synthetic_dense(70, hp, dtype)
+    orc = oracle_decoder(oracle, hp, tens, ctx_len=32)
+    dec = qh.Decoder(hp, tens, ctx_len=32)
+    ids = np.random.default_rng(4).integers(0, hp.vocab_size, 3).astype(np.int32)
+    _steps_vs_oracle(oracle, orc, dec, ids, 3, shortlist=False)
+    dec.close()
