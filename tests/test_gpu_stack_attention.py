@@ -1,6 +1,7 @@
 """GPU parity of the prefill stack's attention (qh_attn.hip) where its launches change: rows on both sides of the one-launch
-limit, pair groups that end in the middle, every head grouping, contexts that are no multiple of a cache block, a stack
-larger than the score workspace, and values that overflow to infinity. The reference side is the same decoder at its
+limit and of the sizes where the number of workgroups decides, pair groups that end in the middle, 1, 2, 3, 4 and 7 query
+heads to a KV head, contexts that are no multiple of a cache block, a stack larger than the score workspace or with a
+smaller one, and infinite values and keys. The reference side is the same decoder at its
 default 32-token chunks (attention_kernel, itself compared with the oracle in test_gpu_decoder.py and test_gpu_options.py):
 states, logits and every cache row must be equal bit for bit."""
 import numpy as np
@@ -62,19 +63,92 @@ def test_stack_attention_larger_than_its_workspace(qh, gpu):
     _compare(qh, hp, qnt.synthetic_q4mix(7, hp, shortlist=False), 8192, 1024, (5600,))
 
 
-@pytest.mark.parametrize("turns", [(300,), (1500,)])
-def test_stack_attention_infinite_values(qh, gpu, turns):
-    """Value projections large enough that some rows overflow f16: an infinite value of a later token must not reach an
-    earlier one (0 times it is NaN), so the second layer's cache rows stay equal."""
-    qnt = qnt_module()
+_OUTLIER = 511  # the token whose rows overflow
+
+
+def _outlier_model(qnt, kind):
+    """A two-layer model in which one token, and no other, has an infinite value (kind "value": dimension 7) or key
+    (dimension 31, which RoPE hardly turns at these positions): its embedding is 0 but for one dimension, which every
+    other token has 0 in, and one projection row weighs that dimension with 5,080 (normed it is 16; f16 ends at 65,504).
+    "key_low": every head's q is negative there, the score -inf; "key_high": positive, +inf; "key_nan": a second infinite
+    dimension with the other sign, NaN."""
     hp = qnt.HParams(vocab_size=512, dim=256, n_layers=2, n_heads=4, n_kv_heads=1, head_dim=64, ffn_dim=512)
     tens = qnt.synthetic_q4mix(9, hp, shortlist=False)
-    rec = tens["model.layers.0.self_attn.v_proj.weight"]
-    data = np.array(rec.data)
-    scales = data[rec.rows * rec.cols:].view(np.float16)
-    scales[:] = (scales.astype(np.float32) * 3e5).astype(np.float16)  # |v| reaches 65,504 at a few positions
-    tens["model.layers.0.self_attn.v_proj.weight"] = qnt.TensorRec(rec.dtype, rec.rows, rec.cols, data)
-    _compare(qh, hp, tens, 1600, 512, turns)
+
+    def edit(name):
+        rec = tens[name]
+        data = np.array(rec.data)
+        tens[name] = qnt.TensorRec(rec.dtype, rec.rows, rec.cols, data, rec.ndim)
+        return data[:rec.rows * rec.cols].view(np.int8).reshape(rec.rows, rec.cols), \
+            data[rec.rows * rec.cols:].view(np.float16).reshape(rec.rows, rec.cols // 32)
+
+    codes, scales = edit("model.embed_tokens.weight")
+    codes[:, 5] = 0
+    codes[_OUTLIER] = 0
+    codes[_OUTLIER, 5], scales[_OUTLIER, 0] = 127, 0.02
+    p = "model.layers.0.self_attn."
+    codes, scales = edit(p + ("v" if kind == "value" else "k") + "_proj.weight")
+    for r in (7,) if kind == "value" else (31,) if kind != "key_nan" else (31, 30):
+        codes[r, :32], codes[r, 5], scales[r, 0] = 0, 127, 40.0
+    if kind != "value":
+        rec = tens[p + "q_proj.bias"]
+        bias = np.array(rec.data).view(np.float32).copy()
+        bias.reshape(4, 64)[:, 31] = -4.0 if kind == "key_low" else 4.0
+        bias.reshape(4, 64)[:, 30] = -4.0
+        tens[p + "q_proj.bias"] = qnt.TensorRec(rec.dtype, rec.rows, rec.cols, bias.view(np.uint8), rec.ndim)
+    return hp, tens
+
+
+@pytest.mark.parametrize("kind", ["value", "key_low", "key_high", "key_nan"])
+@pytest.mark.parametrize("turns,at", [
+    ((300,), (201, 202, 203, 255)),         # four tokens of a head to a workgroup
+    ((900,), (801, 802, 803, 863)),         # 16 pairs (four tokens) to a workgroup
+    ((900, 400), (1101, 1102, 1103, 1215)),  # 64 pairs (16 tokens) to a group, three launches
+])
+def test_stack_attention_infinite_values(qh, gpu, turns, at, kind):
+    """One infinite value or key, at a position inside a workgroup's or group's tokens and inside a step of four rows, or
+    the last row of a tile: it must not reach a token before it (0 times it is NaN), whose second-layer cache rows stay
+    those of a prompt without it. A score of -inf has the weight 0, so that later tokens' rows stay finite too; after the
+    others they are NaN. Equal to the 32-token chunks bit for bit."""
+    qnt = qnt_module()
+    hp, tens = _outlier_model(qnt, kind)
+    n = sum(turns)
+    plain = np.random.default_rng(3).integers(0, _OUTLIER, n).astype(np.int32)
+    decs = []
+    for stack in (32, 1024):
+        dec = qh.Decoder(hp, tens, ctx_len=1408)
+        dec.set_prefill_stack(stack)
+        decs.append(dec)
+
+    def run(dec, ids):
+        pos = 0
+        for m in turns:
+            dec.prefill(ids[pos:pos + m], pos, top_k=0)
+            pos += m
+        return [c.view(np.float16) for l in range(2) for c in dec.kv(l, n)]
+
+    base = run(decs[1], plain)
+    assert all(np.isfinite(c).all() for c in base)
+    for p in at:
+        ids = plain.copy()
+        ids[p] = _OUTLIER
+        want, got = run(decs[0], ids), run(decs[1], ids)
+        inf0 = ~np.isfinite(want[1] if kind == "value" else want[0])  # layer 0: infinite there and nowhere else
+        assert inf0[p].any() and not np.delete(inf0, p, 0).any()
+        for w, b in zip(want[2:], base[2:]):  # layer 1
+            assert (w[:p] == b[:p]).all() and np.isfinite(w[:p]).all()
+            assert np.isfinite(w[p:]).all() if kind == "key_low" else np.isnan(w[p:]).any(1).all()
+        for w, g in zip(want, got):
+            assert _equal(w.view(np.uint16), g.view(np.uint16)), p
+    for dec in decs:
+        dec.close()
+    q = tens["model.layers.0.self_attn.q_proj.weight"]  # layer 1 does depend on layer 0's attention
+    tens["model.layers.0.self_attn.q_proj.weight"] = qnt.TensorRec(q.dtype, q.rows, q.cols, np.zeros_like(q.data))
+    dec = qh.Decoder(hp, tens, ctx_len=1408)
+    dec.set_prefill_stack(1024)
+    other = run(dec, plain)
+    dec.close()
+    assert (other[2][2:] != base[2][2:]).any(1).mean() > 0.99
 
 
 @pytest.mark.parametrize("n_heads,n_kv,head_dim,ctx,stack,turns", [
