@@ -1070,7 +1070,10 @@ MmPlan matmul_plan(int rows, int cols, int n) {
         // CUs, smaller chunks let several workgroups share a CU: four waves with 8-block chunks up to two tiles per CU
         // (Q4_0 896x4864 at M = 1024: 37.3 us, 45.2 with eight waves, 39.3 with 4-block chunks; 1536x8960 at 512:
         // 62.9, 73.6, 66.9), 4-block chunks beyond (4096x14336 at 300: 138.6, 165.9 with eight waves, 151.1 with 8-block
-        // chunks; Q8_0 4096x4096 at 700: 74.8, 106.9, 87.5), as on short rows.
+        // chunks; Q8_0 4096x4096 at 700: 74.8, 106.9, 87.5), as on short rows. The last is also what gate / up with the
+        // SwiGLU epilogue takes (launch_matmul_swiglu), so on a stack of a model of 2,048 columns and more they are one
+        // launch from two tiles per CU on: gate, up, SwiGLU and down of 5,632 Q4_0 rows by 2,048 at 512 tokens 170 -> 117
+        // us against eight waves and a SwiGLU launch, of 14,336 by 4,096 at 256 367 -> 283.
         const long cus = device_cus();
         if (cols >= 2048 && tiles32 <= cus) return MmPlan{false, 1, 8, false, 0, true, 16, 32};
         return MmPlan{false, 1, 4, false, 0, true, cols >= 2048 && tiles32 <= 2 * cus ? 8 : 4, 32};

@@ -209,3 +209,17 @@ def test_stack_with_a_smaller_score_workspace(qh, gpu):
         dec.close()
     assert _equal(got[0][0], got[1][0])
     assert all(_equal(a, b) for a, b in zip(got[0][1], got[1][1]))
+
+
+@pytest.mark.parametrize("dtype", [2, 3])
+def test_wide_model_stack_equals_chunks(qh, gpu, dtype):
+    """Rows of 2,048 with more than two 64 x 32 tiles per CU: the prompt matmul's plan with 4-block chunks, which on a stack
+    also takes gate and up with SwiGLU in the epilogue, in whole and ragged token tiles."""
+    qnt = qnt_module()
+    import quanta_cpp_amd.synth as synth
+    hp = qnt.HParams(vocab_size=512, dim=2048, n_layers=1, n_heads=32, n_kv_heads=8, head_dim=64, ffn_dim=4352)
+    tens = qnt.synthetic_q4mix(19, hp, shortlist=False)
+    if dtype == 2:
+        for i, (n, r, c) in enumerate((("gate", 4352, 2048), ("up", 4352, 2048), ("down", 2048, 4352))):
+            tens["model.layers.0.mlp.%s_proj.weight" % n] = qnt.TensorRec(2, r, c, synth.q8_tensor(900 + i, r, c))
+    _compare(qh, hp, tens, 320, 160, (160, 131))
