@@ -321,15 +321,7 @@ __device__ __forceinline__ float dev_expf(float x, const uint64_t* lds_tab) { re
 // The same for x <= 0 or NaN (a score minus the maximum), without its branches, so that a lane's exponentials
 // interleave: the general path for every x, then the two results that differ, 0 below the underflow bound and the NaN.
 __device__ __forceinline__ float dev_expf_nonpos(float x, const uint64_t* lds_tab) {
-    using namespace expf_detail;
-    const double xd = (double)x;
-    double kd = __builtin_fma(kInvLn2N, xd, kShift);
-    const uint64_t ki = __builtin_bit_cast(uint64_t, kd);
-    kd -= kShift;
-    const double r = __builtin_fma(kInvLn2N, xd, -kd), r2 = r * r;
-    const double s = __builtin_bit_cast(double, lds_tab[ki % 32] + (ki << 47));
-    const double z = __builtin_fma(kC0, r, kC1);
-    const float y = (float)(__builtin_fma(z, r2, __builtin_fma(kC2, r, 1.0)) * s);
+    const float y = expf_detail::general<2>(x, lds_tab);
     return x != x ? x + x : x < -0x1.9fe368p6f ? 0.0f : y;
 }
 

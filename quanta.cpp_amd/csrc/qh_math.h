@@ -58,21 +58,13 @@ QH_HD inline double from_bits_f64(uint64_t u) {
     return d;
 }
 
-}  // namespace expf_detail
-
+// expf where the result neither overflows nor is infinite or NaN (x not NaN, at most 0x1.62e42ep6f); below
+// -0x1.9fe368p6f, where it is 0, the result means nothing.
 // FUSED: 0 = no multiply-add fused, 1 = the polynomial's three multiply-adds fused, 2 = also x * 32/ln2 fused
 // into the rounding shift and the reduction.
 // tab: the 32-entry table (kTab, or a copy of it, e.g. in LDS).
 template <int FUSED>
-QH_HD inline float expf_variant(float x, const uint64_t* tab = expf_detail::kTab) {
-    using namespace expf_detail;
-    const uint32_t abstop = (bits_f32(x) >> 20) & 0x7ffu;
-    if (abstop >= (bits_f32(88.0f) >> 20)) {
-        if (bits_f32(x) == 0xff800000u) return 0.0f;           // -inf
-        if (abstop >= (bits_f32(__builtin_inff()) >> 20)) return x + x;  // +inf, nan
-        if (x > 0x1.62e42ep6f) return __builtin_inff();       // overflow
-        if (x < -0x1.9fe368p6f) return 0.0f;                   // underflow to +0
-    }
+QH_HD inline float general(float x, const uint64_t* tab) {
     const double xd = (double)x;
     double kd, r;
     if (FUSED >= 2) {
@@ -103,6 +95,21 @@ QH_HD inline float expf_variant(float x, const uint64_t* tab = expf_detail::kTab
     }
     y = y * s;
     return (float)y;
+}
+
+}  // namespace expf_detail
+
+template <int FUSED>
+QH_HD inline float expf_variant(float x, const uint64_t* tab = expf_detail::kTab) {
+    using namespace expf_detail;
+    const uint32_t abstop = (bits_f32(x) >> 20) & 0x7ffu;
+    if (abstop >= (bits_f32(88.0f) >> 20)) {
+        if (bits_f32(x) == 0xff800000u) return 0.0f;           // -inf
+        if (abstop >= (bits_f32(__builtin_inff()) >> 20)) return x + x;  // +inf, nan
+        if (x > 0x1.62e42ep6f) return __builtin_inff();       // overflow
+        if (x < -0x1.9fe368p6f) return 0.0f;                   // underflow to +0
+    }
+    return general<FUSED>(x, tab);
 }
 
 }  // namespace qh
