@@ -1863,6 +1863,14 @@ __global__ __launch_bounds__(1024) void attention_decode_kernel(
     float acc = 0.0f;
     for (int s0 = 0;;) {
         const int se = min(nrows, s0 + kVRows);
+        if (tid >= HD && se < nrows) {  // uniform per wave; pos >= 1 here (a second stage)
+            const int nb8 = (min(nrows, se + kVRows) - se + 7) / 8, lastc = (pos - 1) / 8;
+#pragma unroll
+            for (int u = 0; u < kPre; ++u) {  // units past the stage repeat its last (never stored)
+                const int c = min(tid - HD + kLoaders * u, nb8 * HD - 1);
+                nxt[u] = ld4(vc4 + vchunk(min(se / 8 + c / HD, lastc), c % HD));
+            }
+        }
         if (tid < HD) {
             const_v16f_ptr wp = (const_v16f_ptr)(arow + s0);  // s0 is a multiple of 32: 64-byte aligned
             auto ldv = [&](uint4(&vv)[4], int jr) {  // rows s0 + jr .. + 31 (jr % 32 == 0)
@@ -1919,22 +1927,12 @@ __global__ __launch_bounds__(1024) void attention_decode_kernel(
             } else {
                 use(vA, wA0, wA1, n - jr);
             }
-        } else {  // the other waves
-            if (se < nrows) {  // uniform; pos >= 1 here (a second stage)
-                const int nb8 = (min(nrows, se + kVRows) - se + 7) / 8, lastc = (pos - 1) / 8;
-#pragma unroll
-                for (int u = 0; u < kPre; ++u) {  // units past the stage repeat its last (never stored)
-                    const int c = min(tid - HD + kLoaders * u, nb8 * HD - 1);
-                    nxt[u] = ld4(vc4 + vchunk(min(se / 8 + c / HD, lastc), c % HD));
-                }
-            }
-            if (s0 == 0) {  // 16 lines of the weight row per scalar-load batch
-                const int wi = __builtin_amdgcn_readfirstlane(wave - 1);
-                for (int b = wi * 256; b < nrows; b += (NW - 1) * 256) {
-                    SegWarm warm;
-                    warm.issue(arow + b, nrows - b);
-                    warm.consume();
-                }
+        } else if (s0 == 0) {  // the other waves: 16 lines of the weight row per scalar-load batch
+            const int wi = __builtin_amdgcn_readfirstlane(wave - 1);
+            for (int b = wi * 256; b < nrows; b += (NW - 1) * 256) {
+                SegWarm warm;
+                warm.issue(arow + b, nrows - b);
+                warm.consume();
             }
         }
         s0 = se;
