@@ -217,11 +217,14 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
                 return at_least;
             };
             uint32_t t = 0u, low = 0u;
+            int at_t = n_groups;
             for (int bit = 31; bit >= 0; --bit) {
                 const uint32_t c = t | (1u << bit);
-                t = reach(c) >= k ? c : t;
+                const int at_c = reach(c);
+                t = at_c >= k ? c : t;
+                at_t = at_c >= k ? at_c : at_t;
             }
-            if (reach(t) > k + 8) {  // uniform; within 8 of k the ties add few candidates
+            if (at_t > k + 8) {  // uniform; within 8 of k the ties add few candidates
                 const int need = k - (t == 0xffffffffu ? 0 : reach(t + 1u));  // of the maxima with score T, lowest ids
 #pragma unroll
                 for (int w = 0; w < W; ++w) h[w] = h[w] == t ? (uint32_t)pool[64 * w + lane] : 0u;
