@@ -766,13 +766,13 @@ __device__ uint64_t qh_tl_pa[16];
     do {              \
     } while (0)
 #endif
-template <int HD, int WPE = 1>
+template <int HD, int WPE = 1, bool SINGLE = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void attention_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ bq, const float* __restrict__ bk, const float* __restrict__ bv,
     const float* __restrict__ cs, const int* __restrict__ pos_dev, int ctx, int n_heads, int n_kv,
     uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int8_t* __restrict__ oq, float* __restrict__ od,
-    int* __restrict__ status, float* __restrict__ of, int single) {
+    int* __restrict__ status, float* __restrict__ of) {
     constexpr int HALF = HD / 2, CPR = HD / 8;           // 16-byte chunks per f16 K row
     constexpr int kVRows = (WPE == 1 ? kVStageBytes : 32 * 1024) / (HD * 2);  // V rows one LDS stage holds (mult. of 8)
     constexpr int kVBlk = kVRows / 8;                    // 8-row blocks per stage
@@ -786,17 +786,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     __shared__ uint64_t exptab[32];
     ExpTab et;
     et.load();
-    // single: every token of a prefill stack is its own chunk (token y = blockIdx.y at position *pos_dev + y), its
+    // SINGLE: every token of a prefill stack is its own chunk (token y = blockIdx.y at position *pos_dev + y), its
     // earlier rows all in the cache already (kv_store_kernel), so the workgroup rebuilds only its own row and stores
     // none.
-    const int h = blockIdx.x, y = blockIdx.y, t = single ? 0 : y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int pos0 = *pos_dev + (single ? y : 0), pos = pos0 + t, nrows = pos + 1;
+    const int h = blockIdx.x, y = blockIdx.y, t = SINGLE ? 0 : y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int pos0 = *pos_dev + (SINGLE ? y : 0), pos = pos0 + t, nrows = pos + 1;
     if (pos >= ctx || pos0 < 0) {  // uniform: a step past the context touches no cache row
         if (tid == 0 && h == 0) atomicOr(status, kStatusCtx);
         return;
     }
     const int qd = n_heads * HD, kvd = n_kv * HD, group = n_heads / n_kv, kvh = h / group;
-    if (single) {  // uniform: this token's rows of the projections and of the output
+    if (SINGLE) {  // this token's rows of the projections and of the output
         q += (size_t)y * qd;
         k += (size_t)y * kvd;
         v += (size_t)y * kvd;
@@ -899,7 +899,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     et.store(exptab);
     __syncthreads();
     QH_PASTAMP(1);
-    if (!single && h % group == 0)
+    if (!SINGLE && h % group == 0)
         for (int i = tid; i < HD; i += 256) {
             kc[(kchunk(i >> 3, pos) << 3) + (i & 7)] = kloc[t * HD + i];
             vc[vchunk(pos / 8, i) * 8 + (pos & 7)] = vloc[t * HD + i];
@@ -1196,12 +1196,14 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const float* __restrict__
 // so the register budget is that of two waves per SIMD.
 constexpr int kStackTok = 4;
 constexpr int kStackCtx = 1024;
+template <int HD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void attention_stack_kernel(
     const float* __restrict__ q, const float* __restrict__ bq, const float* __restrict__ cs,
     const int* __restrict__ pos_dev, int n, int ctx, int n_heads, int n_kv, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int8_t* __restrict__ oq, float* __restrict__ od, int* __restrict__ status,
     float* __restrict__ of) {
-    constexpr int HD = 64, HALF = HD / 2, CPR = HD / 8, NTK = kStackTok;
+    static_assert(HD == 64, "a lane per dimension");
+    constexpr int HALF = HD / 2, CPR = HD / 8, NTK = kStackTok;
     constexpr int kVRows = 256, kVBlk = kVRows / 8;  // V rows per LDS stage (32 KB)
     constexpr int kVPer = kVBlk * HD / 256;          // 16-byte V units per thread and stage
     __shared__ __align__(16) float att[NTK][kStackCtx + kChainPad];
@@ -2723,11 +2725,11 @@ hipError_t attention_chunk(Decoder* d, int l, int n, int r0, const int* pos_dev,
     } else if (hp.head_dim == 64) {
         qh_launch((attention_kernel<64, 2>), grid, dim3(256), 0, s, q, k, v, bias(d, l, L_BQ), bias(d, l, L_BK),
                   bias(d, l, L_BV), d->cs, pos_dev, hp.ctx_len, hp.n_heads, hp.n_kv_heads, d->kc + l * layer_k,
-                  d->vc + l * layer_v, oq, od, d->status, of, 0);
+                  d->vc + l * layer_v, oq, od, d->status, of);
     } else {
         qh_launch((attention_kernel<128>), grid, dim3(256), 0, s, q, k, v, bias(d, l, L_BQ), bias(d, l, L_BK),
                   bias(d, l, L_BV), d->cs, pos_dev, hp.ctx_len, hp.n_heads, hp.n_kv_heads, d->kc + l * layer_k,
-                  d->vc + l * layer_v, oq, od, d->status, of, 0);
+                  d->vc + l * layer_v, oq, od, d->status, of);
     }
     return hipGetLastError();
 }
@@ -2754,6 +2756,8 @@ bool few_workgroups(const qh_model_desc& hp, int n, int pos0) {
     return w <= cus && rows <= 2700;
 }
 
+hipError_t attention_few(Decoder* d, int l, int n, uint16_t* kc, uint16_t* vc, hipStream_t s);
+
 // Attention of a prefill stack of n > kChunk tokens at positions *d->pos ..: the f16 cache rows of every token of the
 // stack first (kv_store_kernel), then the stack's (token, head) pairs together (launch_attention_stack), or, where those
 // are few, one workgroup per head and token (each its own chunk, every earlier row read from the cache) or four tokens.
@@ -2770,22 +2774,7 @@ hipError_t attention_stack(Decoder* d, int l, int n, hipStream_t s) {
                   d->cs, d->pos, hp.ctx_len, hp.n_kv_heads, kc, vc);
     QH_TRY(hipGetLastError());
     const int pos0 = d->stack_end - n;
-    if (few_workgroups(hp, n, pos0)) {
-        const dim3 grid(hp.n_heads, n);
-        if (hp.head_dim == 64 && d->stack_end <= kStackCtx)
-            qh_launch(attention_stack_kernel, dim3(hp.n_heads, (n + kStackTok - 1) / kStackTok), dim3(256), 0, s, d->q,
-                      bias(d, l, L_BQ), d->cs, d->pos, n, hp.ctx_len, hp.n_heads, hp.n_kv_heads, kc, vc, d->qb, d->db,
-                      d->status, d->fb);
-        else if (hp.head_dim == 64)
-            qh_launch((attention_kernel<64, 2>), grid, dim3(256), 0, s, d->q, d->k, d->v, bias(d, l, L_BQ),
-                      bias(d, l, L_BK), bias(d, l, L_BV), d->cs, d->pos, hp.ctx_len, hp.n_heads, hp.n_kv_heads, kc, vc,
-                      d->qb, d->db, d->status, d->fb, 1);
-        else
-            qh_launch((attention_kernel<128>), grid, dim3(256), 0, s, d->q, d->k, d->v, bias(d, l, L_BQ),
-                      bias(d, l, L_BK), bias(d, l, L_BV), d->cs, d->pos, hp.ctx_len, hp.n_heads, hp.n_kv_heads, kc, vc,
-                      d->qb, d->db, d->status, d->fb, 1);
-        return hipGetLastError();
-    }
+    if (few_workgroups(hp, n, pos0)) return attention_few(d, l, n, kc, vc, s);
     AttnStack a{};
     a.q = d->q;
     a.bq = bias(d, l, L_BQ);
@@ -3272,5 +3261,30 @@ hipError_t decoder_set_sampler(Decoder* d, const qh_sampler_params* p, uint64_t 
     const uint64_t st = seed | 1u;  // Sampler's constructor (sampler.cpp:10-13)
     return hipMemcpy(d->rng, &st, sizeof st, hipMemcpyHostToDevice);
 }
+
+namespace {
+
+// A stack of few workgroups (few_workgroups), its cache rows stored. Last in the file, its kernels templates, so that the
+// kernels of a decode step keep their places in the code: behind these kernels 16 steps of two layers at position 3,500
+// took 1,915 us, not 1,893.
+hipError_t attention_few(Decoder* d, int l, int n, uint16_t* kc, uint16_t* vc, hipStream_t s) {
+    const qh_model_desc& hp = d->hp;
+    const dim3 grid(hp.n_heads, n);
+    if (hp.head_dim == 64 && d->stack_end <= kStackCtx)
+        qh_launch((attention_stack_kernel<64>), dim3(hp.n_heads, (n + kStackTok - 1) / kStackTok), dim3(256), 0, s, d->q,
+                  bias(d, l, L_BQ), d->cs, d->pos, n, hp.ctx_len, hp.n_heads, hp.n_kv_heads, kc, vc, d->qb, d->db,
+                  d->status, d->fb);
+    else if (hp.head_dim == 64)
+        qh_launch((attention_kernel<64, 2, true>), grid, dim3(256), 0, s, d->q, d->k, d->v, bias(d, l, L_BQ),
+                  bias(d, l, L_BK), bias(d, l, L_BV), d->cs, d->pos, hp.ctx_len, hp.n_heads, hp.n_kv_heads, kc, vc, d->qb,
+                  d->db, d->status, d->fb);
+    else
+        qh_launch((attention_kernel<128, 1, true>), grid, dim3(256), 0, s, d->q, d->k, d->v, bias(d, l, L_BQ),
+                  bias(d, l, L_BK), bias(d, l, L_BV), d->cs, d->pos, hp.ctx_len, hp.n_heads, hp.n_kv_heads, kc, vc, d->qb,
+                  d->db, d->status, d->fb);
+    return hipGetLastError();
+}
+
+}  // namespace
 
 }  // namespace qh
