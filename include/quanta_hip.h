@@ -251,18 +251,21 @@ uint64_t qh_sampler_state(uint64_t seed);
  *                      ids whose logits are finite; NULL / NULL to consider every id below n_valid.
  *   history[0, n_hist): DEVICE token history (the session's prompt and generated ids), NULL when n_hist is 0.
  * Requires 1 <= n_valid <= QH_SAMPLE_MAX_VOCAB and, with temperature > 0, min(top_k or n_valid, n_valid) <=
- * QH_SAMPLE_MAX_TOPK (qh_sample_ws takes any number). Ties between equal logits in the top-k go to the lower id
+ * QH_SAMPLE_MAX_TOPK (qh_sample_ws takes any number, and over full logits of tens of thousands of ids is several times
+ * as fast for any top_k). Ties between equal logits in the top-k go to the lower id
  * (unspecified in the reference).
  * Replaces: Sampler::sample (reference sampler.cpp:22-85) and Sampler's generator (sampler.cpp:10-21). */
 int qh_sample(const float* logits, int32_t n_valid, const int32_t* rows, const qh_head_stats* head_stats,
               const int32_t* history, int32_t n_hist, const qh_sampler_params* params, uint64_t* state,
               int32_t* out_id, void* stream);
 
-/* qh_sample with a DEVICE workspace of qh_sample_workspace_bytes(n_valid) bytes (16-byte aligned), which lifts the
- * QH_SAMPLE_MAX_TOPK limit: any top_k, top_k 0 (every id a survivor) included. More survivors than that are sorted by
- * a device-wide radix sort (4 passes over the logit half); the softmax sum, top-p, total and draw then run in the
- * reference's order and stop where the remaining terms can no longer change a rounded result. Calls that share a
- * workspace must not overlap. Replaces: Sampler::sample (reference sampler.cpp:22-85) with top_k 0 or large. */
+/* qh_sample with a DEVICE workspace of qh_sample_workspace_bytes(n_valid) bytes (16-byte aligned). Over full logits
+ * (rows NULL) of 8,192 ids and more the whole GPU first finds the largest of each group of 256 ids, and one workgroup
+ * then reads only the groups that can hold a survivor: 151,936 ids at top_k 20 take 20 us, 72 without a workspace
+ * (greedy draws from 16,384 ids on: 6 and 32). It also lifts the QH_SAMPLE_MAX_TOPK limit: any top_k, top_k 0 (every id
+ * a survivor) included. More survivors than that are sorted by a device-wide radix sort (4 passes over the logit half);
+ * the softmax sum, top-p, total and draw then run in the reference's order and stop where the remaining terms can no
+ * longer change a rounded result. Any call may write the workspace: calls that share one must not overlap. Replaces: Sampler::sample (reference sampler.cpp:22-85) with top_k 0 or large. */
 size_t qh_sample_workspace_bytes(int32_t n_valid);
 int qh_sample_ws(const float* logits, int32_t n_valid, const int32_t* rows, const qh_head_stats* head_stats,
                  const int32_t* history, int32_t n_hist, const qh_sampler_params* params, uint64_t* state,
@@ -352,10 +355,13 @@ int qh_decoder_views(qh_decoder* d, qh_decoder_state* v);
 /* The prefill stack: how many prompt tokens later qh_decoder_prefill calls take through each layer's norms and
  * matmuls at once. 32 (the default) is the reference's chunk (Model::kBatch, model.h:52; forward_batch,
  * model.cpp:349-361); a multiple of 32 up to 1024 runs the same arithmetic on larger batches (the matmul tile kernels
- * at M up to `stack`), attention still in 32-token sub-chunks in order, so every hidden state, cache row and logit is
- * bit-identical to the 32-token chunks. Reallocates the decoder's work buffers: it synchronises the device, the
- * pointers qh_decoder_views gave (xq / xd) change and their contents are lost, and a step captured in a HIP graph
- * before the call must be captured again. On failure the previous stack stays.
+ * at M up to `stack`; attention of the whole stack at once over an fp16 cache, in 32-token sub-chunks in order over an
+ * f32 one), so every hidden state, cache row and logit is bit-identical to the 32-token chunks. Reallocates the
+ * decoder's work buffers: it synchronises the device, the pointers qh_decoder_views gave (xq / xd) change and their
+ * contents are lost, and a step captured in a HIP graph before the call must be captured again. With an fp16 cache of
+ * more than 1,024 positions a stack above 32 also takes a workspace for attention scores: 264 bytes per position, KV
+ * head and group of 64 (token, query head) pairs of it, at most 256 MB, and less (down to one such group) where memory
+ * is short, in more passes. On failure the previous stack stays.
  * Replaces: nothing (the reference's chunk is a compile-time constant); a scheduling choice of the GPU path. */
 int qh_decoder_set_prefill_stack(qh_decoder* d, int stack);
 

@@ -277,8 +277,9 @@ def sample(logits, params: qh_sampler_params, state, history=None, n_valid: int 
            ws=None):
     """One Sampler::sample draw on the device: returns the chosen id as a device int32 tensor of one element.
     state: device uint64 tensor of one element (advanced in place); history: device int32 tensor or None;
-    head: a ShortlistHead whose last call's row list and stats restrict the candidates; ws: a device uint8 tensor of
-    sample_workspace_bytes(n_valid) bytes for more than SAMPLE_MAX_TOPK survivors (qh_sample_ws), or None."""
+    head: a ShortlistHead whose last call's row list and stats restrict the candidates; ws: a sample_workspace(n_valid)
+    (qh_sample_ws), or None. Draws over full logits take a fraction of the time with one (151,936 ids, top-k 20: 20 us
+    against 72), and more than 256 survivors of the top-k need one; calls that share one must not overlap."""
     torch = _torch()
     out = torch.empty(1, dtype=torch.int32, device=logits.device)
     nv = logits.numel() if n_valid is None else n_valid
@@ -439,8 +440,8 @@ class Decoder:
             pass
 
     def set_prefill_stack(self, stack: int):
-        """Prompt tokens per launch of each layer's norms and matmuls (32 = the reference's chunk; up to 1024), with
-        bit-identical results; the device views are re-read (the work buffers move)."""
+        """Prompt tokens per launch of each layer's norms, matmuls and (f16 cache) attention (32 = the reference's chunk;
+        up to 1024), with bit-identical results; the device views are re-read (the work buffers move)."""
         _check(lib().qh_decoder_set_prefill_stack(self.h, stack))
         st = qh_decoder_state()
         _check(lib().qh_decoder_views(self.h, C.byref(st)))

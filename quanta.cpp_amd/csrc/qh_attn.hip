@@ -21,8 +21,10 @@
 // bytes are its operand of four 16x16x4 products.
 //
 // Measured per layer (14 heads, 2 KV heads, head_dim 64) against one token to a wave, lane per position for the scores
-// and per dimension for the outputs, weights as LDS broadcasts: 512 tokens 35 -> 26 us, 1,024 tokens 108 -> 55 us;
-// 1,024 tokens at position 1,024 576 -> 127 us, 952 at 2,048 811 -> 170 us (scores 60, softmax 50, values 60).
+// and per dimension for the outputs, weights as LDS broadcasts: 512 tokens 35 -> 24 us (26 before the exponentials lost
+// their branches, which is what the comparisons below were measured against), 1,024 tokens 108 -> 55 us; 1,024 tokens at
+// position 1,024 576 -> 127 us, 952 at 2,048 811 -> 170 us (scores 60, softmax 50, values 60). Stacks of few workgroups
+// go elsewhere (few_workgroups, qh_decoder.hip).
 #include "qh_device.h"
 #include "qh_internal.h"
 
@@ -430,7 +432,7 @@ __global__ __launch_bounds__(256) void attn_values_kernel(AttnStack a, int ng) {
 // HD / 4 of the output dimensions. Keys and values come straight from the cache as whole 16-byte units, the next unit's
 // load in flight, four lanes to a unit, each selecting its two halves (as 4-byte loads, which the address unit serves
 // no faster, 512 tokens took 39 us against 26). Serial latency bounds it: 8 or 16 waves a workgroup measured no faster.
-// At 64 to 1,024 rows it is ahead of the three launches (512 tokens 26 against 32 us and two launches, 1,024 tokens 55
+// Up to 1,024 rows it is ahead of the three launches (512 tokens 26 against 32 us and two launches, 1,024 tokens 55
 // against 70, 64 tokens at position 900 equal).
 constexpr int kShortRows = 1024;
 template <int HD>

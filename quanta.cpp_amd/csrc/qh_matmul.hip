@@ -1059,9 +1059,8 @@ MmPlan matmul_plan(int rows, int cols, int n) {
     // 8.4 against 11.9 and 13.3) and eight waves with 16-block chunks on longer rows (Q4_0 896x4864 at M = 512: 22.4,
     // against 23.0 with 8-block chunks, 24.4 with four waves, 25.4 with 16-token workgroups). Long rows with too few
     // 32-token tiles take 16-token workgroups when they make about 192 (896x4864 at M = 256: 19.4 against 24.7
-    // staged). Everywhere else (few tiles) the LDS-staged kernel wins, also over the
-    // register-chain kernel; it measured 4-12% under the LDS and register kernels at 32 tokens (q/k/v, o, gate/up,
-    // down).
+    // staged). Everywhere else (few tiles) the LDS-staged kernel wins, also over the register-chain kernel; it measured
+    // 4-12% under the LDS and register kernels at 32 tokens (q/k/v, o, down).
     const long row_tiles = (rows + 63) / 64;
     const long tiles32 = row_tiles * ((n + 31) / 32), tiles16 = row_tiles * ((n + 15) / 16);
     if (n >= 128 && tiles32 >= 192) {
@@ -1081,8 +1080,11 @@ MmPlan matmul_plan(int rows, int cols, int n) {
     if (n >= 128 && cols >= 2048 && tiles16 >= 192) return MmPlan{false, 1, 4, false, 0, true, 8, 16};
     // Below 128 tokens: 16-token tiles once there are about 192 (Q4_0 4864x896 at 77 tokens 7.6 us, 9.6 staged; 8960x1536 at
     // 40 10.3 and 17.6; 16384x1024 at 20 8.0 and 11.8; Q8_0 12000x2048 at 64 18.6 and 36.7; fewer tiles: 4096x14336 at 20,
-    // 128 of them, 49.4 and 35.6), on long rows the eight waves where they make that many 32-token tiles, at most one per
-    // CU (4096x14336 at 100 tokens 59.0 us, 73.7 with 16-token tiles, 113.0 staged).
+    // 128 of them, 49.4 and 35.6; Q4_0 9728x896 at 32 8.3 and 9.0), on long rows the eight waves where they make that many
+    // 32-token tiles, at most one per CU (4096x14336 at 100 tokens 59.0 us, 73.7 with 16-token tiles, 113.0 staged).
+    // 128 tokens is the line of the sweeps above, not where 16- and 32-token tiles cross: that follows the rounds of
+    // workgroups. Q4_0 4864x896 at 96 tokens 8.4 us, 8.6 with 32-token tiles; 8960x1536 at 97 17.4 and 19.3, at 96 17.3 and
+    // 15.3; 9728x896 at 64 10.1 and 10.3, at 96 13.1 and 11.1, at 127 15.1 and 13.5.
     if (n < 128 && tiles16 >= 192) {
         if (cols >= 2048 && tiles32 >= 192 && tiles32 <= device_cus()) return MmPlan{false, 1, 8, false, 0, true, 16, 32};
         return MmPlan{false, 1, 4, false, 0, true, 8, 16};
