@@ -33,6 +33,8 @@
 #include <type_traits>
 #include <vector>
 
+#include "qh_attn_chunk.h"
+#include "qh_decoder_device.h"
 #include "qh_device.h"
 #include "qh_gemv.h"
 #include "qh_internal.h"
@@ -41,478 +43,6 @@
 namespace qh {
 
 namespace {
-
-constexpr int kChunk = 32;            // prefill chunk (reference Model::kBatch, model.h:52)
-constexpr int kMaxStack = 1024;       // prefill stack limit (tokens whose matmuls share a launch)
-constexpr int kMaxCtx = 8192;         // positions the attention kernel's score array holds
-constexpr int kVStageBytes = 96 * 1024;  // LDS for staged V rows (768 rows at head_dim 64)
-constexpr int kFuseLds = 65536;       // dynamic LDS limit of the fused GEMV kernels
-
-// Positions the V cache holds per layer: the context rounded up to its 8-position blocks.
-inline int v_ctx(int ctx) { return (ctx + 7) & ~7; }
-
-// Floats per attention workgroup's exp row: the context rounded up to 16 (64-byte aligned rows) plus 64 of slack for
-// whole-batch scalar reads past the last position.
-inline int escr_stride(int ctx) { return ((ctx + 15) & ~15) + 64; }
-
-enum { kStatusCtx = 1, kStatusToken = 2 };
-
-
-__device__ __forceinline__ float h2f(uint16_t h) { return f16_to_f32(h); }
-
-// A 16-byte register value as a native vector (register arrays of HIP's uint4 struct are not always split into
-// registers by the compiler; native vectors are).
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ v4u ld4(const void* p) { return *reinterpret_cast<const v4u*>(p); }
-
-// LDS DMA (global_load_lds_dwordx4): lane l's 16 bytes at g go to lds_wave + 16 l, where lds_wave is the same LDS
-// address in every lane of the wave. Counted by vmcnt; the LDS data is valid after s_waitcnt vmcnt(0). Issued in
-// inline assembly, behind the compiler's back: the compiler counts a DMA it knows of as a transfer that may complete
-// out of order, so after one it waits for every outstanding load (vmcnt(0)) before using any earlier load's result
-// and before any LDS access. This way the earlier loads keep their waits, LDS accesses wait for nothing, the caller
-// waits for the transfer itself (s_waitcnt vmcnt(0)) before reading its LDS, and the compiler's waits for loads
-// issued before it become conservative (they also cover the transfers), never short. M0, which the transfer takes
-// its LDS address from, is an input operand of the asm ("{m0}" constraint): the compiler writes it and knows what M0
-// holds afterwards. The s_nop covers the wait state between an M0 write and the transfer that reads it. The body
-// exists only in the device pass (the host pass cannot form an LDS address).
-__device__ __forceinline__ void lds_dma16_async(const void* g, void* lds_wave) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane(
-        (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds_wave);
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(m0) : "memory");
-#endif
-}
-// f32 -> f16 (round to nearest even) of an already rounded f32 value, as the reference stores its f32 K / V results
-// into the f16 cache. The empty asm makes the value opaque, so the compiler cannot fuse the FMA that produced it and
-// this conversion into one v_fma_mixlo_f16, which rounds only once (straight to f16) and differs on double-rounding
-// cases.
-__device__ __forceinline__ uint16_t f2h(float f) {
-    asm volatile("" : "+v"(f));
-    return __builtin_bit_cast(uint16_t, (_Float16)f);
-}
-
-// quantize_q8 of one 32-block held one value per lane of a half-wave (ops_ref.cpp:69-83): the block's absolute
-// maximum / 127, codes rounded half away from zero. Every lane of the half-wave must be active.
-// Maximum over the whole wave (every lane active) with the select o > a ? o : a at each step: DPP within rows of
-// 16, then the gfx950 row swaps (16 and 32 lanes apart).
-__device__ __forceinline__ float wave_max_sel(float a) {
-    auto step = [](float x, float o) { return o > x ? o : x; };
-    a = step(a, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, a), 0xB1, 0xF, 0xF, false)));
-    a = step(a, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, a), 0x4E, 0xF, 0xF, false)));
-    a = step(a, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, a), 0x141, 0xF, 0xF, false)));
-    a = step(a, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, a), 0x140, 0xF, 0xF, false)));
-    uint32_t u = __builtin_bit_cast(uint32_t, a);
-    const auto s16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    a = step(__builtin_bit_cast(float, (uint32_t)s16[0]), __builtin_bit_cast(float, (uint32_t)s16[1]));
-    u = __builtin_bit_cast(uint32_t, a);
-    const auto s32 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    return step(__builtin_bit_cast(float, (uint32_t)s32[0]), __builtin_bit_cast(float, (uint32_t)s32[1]));
-}
-
-// quantize_q8 of the row xs[0, D) (16-byte aligned, D % 32 == 0) into q / d: 8 lanes per block, 32 blocks per pass
-// of 256 threads.
-__device__ __forceinline__ void quant_row_x8(const float* xs, int D, int8_t* __restrict__ q, float* __restrict__ d) {
-    const int nb = D / QK;
-    for (int t = (int)threadIdx.x; t < nb * 8; t += 256) {  // whole 8-lane groups
-        const int b = t >> 3;
-        quant_block_x8(reinterpret_cast<const float4*>(xs)[t], q + b * QK, d + b);
-    }
-}
-
-// acc = op(acc, p[i]) for i = 0 .. n-1 in order, by one thread, over floats in LDS (16-byte aligned, n >= 1). A wave
-// issues about one instruction per 4 cycles whatever its kind, so the loop is shaped for the fewest instructions
-// per element: batches of 32 values read as 8 b128 at immediate offsets from one base, two register sets that
-// alternate without copies (the next batch in flight while the current one is consumed), no clamping. It reads up
-// to kChainPad floats past n: callers size the array n + kChainPad.
-constexpr int kChainPad = 64;
-
-// An LDS address the compiler treats as per-lane: uniform LDS addresses otherwise get rematerialized into a VGPR for
-// every read, costing an instruction each (mbcnt_lo(0, 0) is 0 in every lane).
-template <typename T>
-__device__ __forceinline__ const T* lane_ptr(const T* p) {
-    return p + __builtin_amdgcn_mbcnt_lo(0u, 0u);
-}
-
-template <typename Op>
-__device__ __forceinline__ float lds_chain(const float* p, int n, Op op, float acc0 = 0.0f) {
-    float4 a[8], b[8];
-    auto ld = [](float4(&r)[8], const float* q) {
-        const float4* q4 = reinterpret_cast<const float4*>(q);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) r[k] = q4[k];
-    };
-    float acc = acc0;
-    auto use = [&](const float4(&r)[8], int cnt) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (4 * k + 0 < cnt) acc = op(acc, r[k].x);
-            if (4 * k + 1 < cnt) acc = op(acc, r[k].y);
-            if (4 * k + 2 < cnt) acc = op(acc, r[k].z);
-            if (4 * k + 3 < cnt) acc = op(acc, r[k].w);
-        }
-    };
-    int j = 0;
-    p = lane_ptr(p);
-    ld(a, p);
-    // sched_barrier keeps each prefetch ahead of the values it overlaps (the scheduler would sink it)
-    for (; j + 64 <= n; j += 64) {
-        ld(b, p + j + 32);
-        __builtin_amdgcn_sched_barrier(0);
-        use(a, 32);
-        ld(a, p + j + 64);
-        __builtin_amdgcn_sched_barrier(0);
-        use(b, 32);
-    }
-    if (j + 32 <= n) {
-        ld(b, p + j + 32);
-        __builtin_amdgcn_sched_barrier(0);
-        use(a, 32);
-        use(b, n - j - 32);  // cnt is uniform
-    } else {
-        use(a, n - j);
-    }
-    return acc;
-}
-
-// R float4 per thread of a row of n4 <= 256 R float4 with every load issued before the first use: slot k holds
-// element tid + 256 k (clamped onto the last element, so the loads are unconditional). Kernels take R = row_slots(n4):
-// one load per thread up to D = 1024, eight (D <= 8192) above.
-template <int R>
-struct RowF4 {
-    float4 v[R];
-    __device__ __forceinline__ void load(const float* __restrict__ src, int n4) {
-        const float4* s4 = reinterpret_cast<const float4*>(src);
-#pragma unroll
-        for (int k = 0; k < R; ++k) v[k] = s4[min((int)threadIdx.x + 256 * k, n4 - 1)];
-    }
-};
-constexpr int row_slots(int n4) { return n4 <= 256 ? 1 : 8; }
-
-// ------------------------------------------------------------------------------ segmented sum of squares
-// rmsnorm's sum of squares is one serial chain, ss = fma(x_i, x_i, ss) for i = 0 .. D-1 in order (ops_ref.cpp:195-197):
-// D dependent FMAs, the longest dependency of a decode layer. seg_sum_squares runs it as four segments at once, one
-// per wave, and still returns the chain's value bit for bit:
-//  - wave 0 runs segment 0 from 0;
-//  - the wave of segment k >= 1 runs it from 64 start values at once, one per lane: the f32 rounding of the exact
-//    (double) sum of squares before the segment, and its neighbours 32 below to 31 above in bit order. The chain's
-//    value at the segment start differs from that guess only by the chain's own accumulated rounding (at most 26 ulps
-//    over 2*10^5 random rows of 896, including rows with outliers), so some lane almost always started at exactly
-//    the chain's value, and that lane's result is then the chain's value at the segment end;
-//  - every thread then follows the chain from segment 0 through the lanes whose start matches bit for bit; a value
-//    outside a window (rare) is continued by running that segment serially from it.
-// The chains read x through scalar loads (x is in global memory and no workgroup writes it during the kernel): one
-// 64-byte load feeds 16 FMAs of all 64 lanes with scalar operands, and the LDS stays free for the other waves.
-// Scalar loads can return out of order, so the loop waits for everything outstanding after each 32-value batch,
-// with the next batch already issued; each wave first touches every 64-byte line of its segment (SegWarm) so these
-// loads hit the scalar cache.
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef const __attribute__((address_space(4))) v16f* const_v16f_ptr;
-typedef const __attribute__((address_space(4))) uint32_t* const_u32_ptr;
-
-// lgkmcnt(0) with the vector-memory and export counters left alone (gfx9 s_waitcnt encoding).
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xc07f); }
-
-// acc = fma(g[i], g[i], acc) for i = 0 .. n-1 in order, g uniform across the wave and 64-byte aligned, n % 32 == 0.
-__device__ __forceinline__ float ss_chain_scalar(const float* g, int n, float acc) {
-    const_v16f_ptr p = (const_v16f_ptr)g;
-    const int nv = n / 16;  // even
-    v16f a0 = p[0], a1 = p[1];
-    wait_lgkm0();
-    __builtin_amdgcn_sched_barrier(0);
-    int i = 0;
-#pragma unroll 1
-    for (; i + 4 <= nv; i += 4) {
-        const v16f b0 = p[i + 2], b1 = p[i + 3];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) acc = __builtin_fmaf(a0[k], a0[k], acc);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) acc = __builtin_fmaf(a1[k], a1[k], acc);
-        __builtin_amdgcn_sched_barrier(0);
-        wait_lgkm0();
-        __builtin_amdgcn_sched_barrier(0);
-        a0 = p[min(i + 4, nv - 2)];
-        a1 = p[min(i + 5, nv - 1)];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) acc = __builtin_fmaf(b0[k], b0[k], acc);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) acc = __builtin_fmaf(b1[k], b1[k], acc);
-        __builtin_amdgcn_sched_barrier(0);
-        wait_lgkm0();
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (i + 2 <= nv) {  // nv % 4 == 2: the last batch, loaded by the loop (or before it)
-#pragma unroll
-        for (int k = 0; k < 16; ++k) acc = __builtin_fmaf(a0[k], a0[k], acc);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) acc = __builtin_fmaf(a1[k], a1[k], acc);
-    }
-    return acc;
-}
-
-// One scalar load per 64-byte line of the first 256 values of g[0, n): brings them into the scalar cache; the values
-// are held until consume() so the loads cannot be dropped.
-struct SegWarm {
-    uint32_t v[16];
-    __device__ __forceinline__ void issue(const float* g, int n) {
-        const_u32_ptr q = (const_u32_ptr)g;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = q[min(i * 16, n - 1)];
-    }
-    __device__ __forceinline__ void consume() const {
-        asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]), "s"(v[4]), "s"(v[5]), "s"(v[6]), "s"(v[7]));
-        asm volatile("" ::"s"(v[8]), "s"(v[9]), "s"(v[10]), "s"(v[11]), "s"(v[12]), "s"(v[13]), "s"(v[14]), "s"(v[15]));
-    }
-};
-
-// Sum over the wave of a double, in lane 63 (DPP: pairs, quads, half rows, rows, then rows 0+1 and 2+3 across).
-template <int CTRL, int ROWS = 0xf>
-__device__ __forceinline__ double dpp_f64(double v) {
-    const uint64_t b = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, false);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, false);
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-__device__ __forceinline__ double wave_sum_lane63(double v) {
-    v += dpp_f64<0xb1>(v);         // quad_perm [1,0,3,2]
-    v += dpp_f64<0x4e>(v);         // quad_perm [2,3,0,1]
-    v += dpp_f64<0x141>(v);        // row_half_mirror
-    v += dpp_f64<0x140>(v);        // row_mirror
-    v += dpp_f64<0x142, 0xa>(v);   // row_bcast:15 into rows 1, 3
-    v += dpp_f64<0x143, 0xc>(v);   // row_bcast:31 into rows 2, 3
-    return v;
-}
-
-// acc = op(acc, g[i]) for i = 0 .. n-1 in order (n >= 1), g uniform across the wave and 4-byte aligned. Whole
-// batches of 32 values are read, so up to 32 values past n must be readable.
-template <typename Op>
-__device__ __forceinline__ float chain_scalar(const float* g, int n, float acc, Op op) {
-    const_v16f_ptr p = (const_v16f_ptr)g;
-    const int nb = n >> 5, rem = n & 31;
-    auto use = [&](const v16f& x0, const v16f& x1, int cnt) {  // cnt is uniform
-#pragma unroll
-        for (int k = 0; k < 16; ++k)
-            if (k < cnt) acc = op(acc, x0[k]);
-#pragma unroll
-        for (int k = 0; k < 16; ++k)
-            if (16 + k < cnt) acc = op(acc, x1[k]);
-    };
-    v16f a0 = p[0], a1 = p[1];
-    wait_lgkm0();
-    __builtin_amdgcn_sched_barrier(0);
-    int b = 0;
-#pragma unroll 1
-    for (; b + 2 <= nb; b += 2) {
-        const v16f c0 = p[2 * b + 2], c1 = p[2 * b + 3];
-        __builtin_amdgcn_sched_barrier(0);
-        use(a0, a1, 32);
-        __builtin_amdgcn_sched_barrier(0);
-        wait_lgkm0();
-        __builtin_amdgcn_sched_barrier(0);
-        a0 = p[2 * b + 4];
-        a1 = p[2 * b + 5];
-        __builtin_amdgcn_sched_barrier(0);
-        use(c0, c1, 32);
-        __builtin_amdgcn_sched_barrier(0);
-        wait_lgkm0();
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (b < nb) {  // a full batch in a, the partial one after it
-        const v16f c0 = p[2 * b + 2], c1 = p[2 * b + 3];
-        __builtin_amdgcn_sched_barrier(0);
-        use(a0, a1, 32);
-        __builtin_amdgcn_sched_barrier(0);
-        wait_lgkm0();
-        __builtin_amdgcn_sched_barrier(0);
-        use(c0, c1, rem);
-    } else {
-        use(a0, a1, rem);
-    }
-    return acc;
-}
-
-// Four segments of a chain over n values, wave w running segment w: [0, b1), [b1, b1 + L), [b1 + L, b1 + 2 L),
-// [b1 + 2 L, n).
-struct Segs4 {
-    int b1, L, n;
-    __device__ __forceinline__ int start(int k) const { return k == 0 ? 0 : b1 + (k - 1) * L; }
-    __device__ __forceinline__ int len(int k) const { return k == 0 ? b1 : k == 3 ? n - b1 - 2 * L : L; }
-};
-
-// Workgroup state of one segmented chain.
-struct SegShared {
-    double part[4][4];  // [wave][k]: the wave's share of the exact sum of the chain's terms below segment k's start
-    float res[256];     // every lane's segment result
-    uint32_t gbits[4];  // segment k's guess
-};
-
-// Sums three per-lane partials over the wave into part[wave][1..3]; a barrier must follow before seg_chain_run.
-__device__ __forceinline__ void seg_partials(SegShared& sh, double p1, double p2, double p3) {
-    p1 = wave_sum_lane63(p1);
-    p2 = wave_sum_lane63(p2);
-    p3 = wave_sum_lane63(p3);
-    if ((threadIdx.x & 63) == 63) {
-        const int w = (int)threadIdx.x >> 6;
-        sh.part[w][1] = p1;
-        sh.part[w][2] = p2;
-        sh.part[w][3] = p3;
-    }
-}
-
-// Runs the segments (wave 0 from 0, the wave of segment k from the 64 candidates around its guess), a barrier, then
-// follows the chain through the candidates; returns the chain's end value in every thread. chain(k, start) runs
-// segment k from start in the calling wave (k and start uniform across the wave) and returns its end value. All 256
-// threads call it after the barrier that published part.
-template <typename Chain>
-__device__ __forceinline__ float seg_chain_run(SegShared& sh, Chain chain) {
-    const int tid = (int)threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    float start = 0.0f;
-    if (wave > 0) {
-        const double g = sh.part[0][wave] + sh.part[1][wave] + sh.part[2][wave] + sh.part[3][wave];
-        const uint32_t gb = __float_as_uint((float)g);
-        start = __uint_as_float(gb + (uint32_t)lane - 32u);
-        if (lane == 0) sh.gbits[wave] = gb;
-    }
-    sh.res[tid] = chain(wave, start);
-    __syncthreads();
-    float s = sh.res[0];
-    const uint32_t g1 = sh.gbits[1], g2 = sh.gbits[2], g3 = sh.gbits[3];
-#pragma unroll
-    for (int k = 1; k < 4; ++k) {
-        const uint32_t j = __float_as_uint(s) - (k == 1 ? g1 : k == 2 ? g2 : g3) + 32u;
-        if (j < 64u)
-            s = sh.res[64 * k + j];
-        else
-            s = chain(k, s);
-    }
-    return s;
-}
-
-// The chain's value ss of x[0, D) in every thread: segments [0, S0) and three of L = (D / 4) rounded down to a
-// multiple of 32 (S0 = D - 3 L >= L). x: global, 64-byte aligned, not written during the kernel; xr: this thread's
-// RowF4 of x; warm: seg_warm(x, D), issued by the same thread. All 256 threads of the workgroup call it (two barriers
-// inside). D % 64 == 0, 128 <= D <= 8192.
-__device__ __forceinline__ Segs4 seg_split(int D) {
-    const int L = (D / 4) & ~31;
-    return Segs4{D - 3 * L, L, D};
-}
-// The scalar loads that bring this wave's segment of x into the scalar cache (issued early, consumed by
-// seg_sum_squares).
-__device__ __forceinline__ SegWarm seg_warm(const float* __restrict__ x, int D) {
-    const Segs4 sg = seg_split(D);
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    SegWarm warm;
-    warm.issue(x + sg.start(wave), sg.len(wave));
-    return warm;
-}
-template <int R>
-__device__ float seg_sum_squares(const float* __restrict__ x, int D, const RowF4<R>& xr, const SegWarm& warm,
-                                 int tlk = -1) {
-    (void)tlk;
-    __shared__ SegShared sh;
-    const int tid = (int)threadIdx.x, n4 = D / 4;
-    const Segs4 sg = seg_split(D);
-    double p1 = 0.0, p2 = 0.0, p3 = 0.0;
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const int i4 = tid + 256 * k;
-        if (i4 < n4) {
-            const float4 v = xr.v[k];
-            const double s = (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w;
-            const int e = 4 * i4;
-            p1 += e < sg.start(1) ? s : 0.0;
-            p2 += e < sg.start(2) ? s : 0.0;
-            p3 += e < sg.start(3) ? s : 0.0;
-        }
-    }
-    seg_partials(sh, p1, p2, p3);
-    __syncthreads();
-    QH_WSTAMP(tlk, 4);
-    warm.consume();
-    const float r = seg_chain_run(sh, [&](int k, float s0) { return ss_chain_scalar(x + sg.start(k), sg.len(k), s0); });
-    QH_WSTAMP(tlk, 5);
-    return r;
-}
-
-// seg_sum_squares for a row held in LDS (xs, complete, 16-byte aligned, kChainPad floats of slack; written in this
-// kernel, so not readable through scalar loads): the same segments and candidate starts, each segment's chain reading
-// its operands from LDS (the four waves' broadcast reads slow each other, ~12 cycles per element, against ~6 for
-// scalar operands, still a quarter of the serial chain). xr: this thread's RowF4 of the row's values. All 256 threads
-// call it (two barriers inside).
-template <int R>
-__device__ float seg_sum_squares_lds(const float* xs, int D, const RowF4<R>& xr) {
-    __shared__ SegShared sh;
-    const int tid = (int)threadIdx.x, n4 = D / 4;
-    const Segs4 sg = seg_split(D);
-    double p1 = 0.0, p2 = 0.0, p3 = 0.0;
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const int i4 = tid + 256 * k;
-        if (i4 < n4) {
-            const float4 v = xr.v[k];
-            const double s = (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w;
-            const int e = 4 * i4;
-            p1 += e < sg.start(1) ? s : 0.0;
-            p2 += e < sg.start(2) ? s : 0.0;
-            p3 += e < sg.start(3) ? s : 0.0;
-        }
-    }
-    seg_partials(sh, p1, p2, p3);
-    __syncthreads();
-    return seg_chain_run(sh, [&](int k, float s0) {
-        return lds_chain(xs + sg.start(k), sg.len(k), [](float acc, float v) { return __builtin_fmaf(v, v, acc); }, s0);
-    });
-}
-
-// rmsnorm scale 1 / sqrt(ss / D + eps) (ops_ref.cpp:197-198).
-__device__ __forceinline__ float rms_scale(float ss, int D, float eps) {
-    return 1.0f / __builtin_sqrtf(ss / (float)D + eps);
-}
-
-// The sum of squares of xs[0, D) (LDS, complete, kChainPad floats of slack) by thread 0, in every thread.
-__device__ __forceinline__ float lds_sum_squares(const float* xs, int D) {
-    __shared__ float ss_sh;
-    if (threadIdx.x == 0) ss_sh = lds_chain(xs, D, [](float acc, float v) { return __builtin_fmaf(v, v, acc); });
-    __syncthreads();
-    return ss_sh;
-}
-
-// y = x * scale * w of the row xs[0..D) (LDS; each thread reads and rewrites its own float4s, slot k = tid + 256 k),
-// also to `normed` when given, then quantize_q8 of y. All 256 threads call it; xs is free after its return only
-// after a barrier.
-template <int R>
-__device__ void normalize_quant_lds(float* xs, int D, float scale, const RowF4<R>& wr, int8_t* __restrict__ oq,
-                                    float* __restrict__ od, float* __restrict__ normed) {
-    const int tid = (int)threadIdx.x, n4 = D / 4;
-    float4* x4 = reinterpret_cast<float4*>(xs);
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const int i4 = tid + 256 * k;
-        if (i4 < n4) {
-            float4 xv = x4[i4];
-            xv.x = xv.x * scale * wr.v[k].x;
-            xv.y = xv.y * scale * wr.v[k].y;
-            xv.z = xv.z * scale * wr.v[k].z;
-            xv.w = xv.w * scale * wr.v[k].w;
-            x4[i4] = xv;
-            if (normed) reinterpret_cast<float4*>(normed)[i4] = xv;
-        }
-    }
-    __syncthreads();
-    quant_row_x8(xs, D, oq, od);
-}
-
-// rmsnorm of the row xs[0..D) (LDS, 16-byte aligned, complete) with weight w (loaded into wr by the caller before
-// the row was complete, so its latency is hidden), then quantize_q8 of the normed row; also written to `normed`
-// when given (ops_ref.cpp:195-199: ss += x*x as one FMA per element in order, scale = 1/sqrt(ss/n + eps),
-// y = x * scale * w). Called by all 256 threads of a workgroup; D % 64 == 0, D <= 8192.
-template <int R>
-__device__ void norm_quant_lds(float* xs, int D, const RowF4<R>& wr, float eps, int8_t* __restrict__ oq,
-                               float* __restrict__ od, float* __restrict__ normed) {
-    normalize_quant_lds(xs, D, rms_scale(lds_sum_squares(xs, D), D, eps), wr, oq, od, normed);
-}
 
 // Activation fill for a GEMV tile whose input is rmsnorm(x) * w quantized (the decode step's q/k/v and gate/up
 // inputs): every workgroup normalises the residual row itself, while its first pass of weight loads is in flight,
@@ -740,412 +270,6 @@ __global__ __launch_bounds__(256) void add_rmsnorm_quant_kernel(float* __restric
                         normed ? normed + (size_t)t * D : nullptr);
 }
 
-// Attention of token t (position pos0 + t) and query head h over positions [0, pos0 + t], for a chunk of n <= 32
-// tokens whose raw projections are q [n][n_heads*HD], k / v [n][n_kv*HD]. One workgroup per (head, token).
-// Cache layouts (f16 bits, per layer): K in 16-byte chunks of 8 dimensions, [n_kv][HD/8][ctx][8], so the lanes of a
-// wave that read chunk c of 64 consecutive positions read 1 KB of contiguous memory (one row per lane, each lane's
-// row complete after HD/8 reads); V in blocks of 8 positions, [pos/8][n_kv*HD][8], so one 16-byte read gives a lane 8
-// consecutive positions of its dimension. Rows below pos0 come from the cache; the
-// chunk's own rows are rebuilt from k / v (bias, RoPE, f16 rounding, exactly as stored), and workgroups of the first
-// query head of each KV group store their token's row. The output (HD values) is quantized straight into oq / od
-// ([n][n_heads*HD] codes, one scale per 32 values).
-// WPE = 1: a 96 KB V stage, one workgroup per CU (one wave per SIMD, which lets the compiler keep three cached K rows
-// per thread in registers). WPE = 2 (prefill chunks at head_dim 64): a 32 KB stage (256 rows) and two cached K rows
-// per thread, so two workgroups share a CU (LDS under 80 KB, registers under 256 each) and the 448 workgroups of a
-// 14-head chunk run in one round instead of two; their serial chains leave each SIMD mostly idle.
-// Timeline stamps of the chunk's last token, query head 0 (compiled in only with -DQH_TIMELINE; the last launch's
-// stamps stay in qh_tl_pa, qh_timeline_pa_read copies them out).
-#if defined(QH_TIMELINE)
-__device__ uint64_t qh_tl_pa[16];
-#define QH_PASTAMP(i)                                                                                        \
-    do {                                                                                                     \
-        if (blockIdx.x == 0 && blockIdx.y == gridDim.y - 1 && threadIdx.x == 0) qh_tl_pa[i] = __builtin_readcyclecounter(); \
-    } while (0)
-#else
-#define QH_PASTAMP(i) \
-    do {              \
-    } while (0)
-#endif
-template <int HD, int WPE = 1, bool SINGLE = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void attention_kernel(
-    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    const float* __restrict__ bq, const float* __restrict__ bk, const float* __restrict__ bv,
-    const float* __restrict__ cs, const int* __restrict__ pos_dev, int ctx, int n_heads, int n_kv,
-    uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int8_t* __restrict__ oq, float* __restrict__ od,
-    int* __restrict__ status, float* __restrict__ of) {
-    constexpr int HALF = HD / 2, CPR = HD / 8;           // 16-byte chunks per f16 K row
-    constexpr int kVRows = (WPE == 1 ? kVStageBytes : 32 * 1024) / (HD * 2);  // V rows one LDS stage holds (mult. of 8)
-    constexpr int kVBlk = kVRows / 8;                    // 8-row blocks per stage
-    __shared__ __align__(16) float att[kMaxCtx + kChainPad];
-    __shared__ __align__(16) uint4 vst[(kVBlk + 4) * HD];  // [block][dim] -> 8 rows; 4 blocks of read padding
-    __shared__ __align__(16) uint16_t kloc[kChunk * HD];
-    __shared__ __align__(16) uint16_t vloc[kChunk * HD];
-    __shared__ __align__(16) float qs[HD];
-    __shared__ float red[4];
-    __shared__ float sum_sh;
-    __shared__ uint64_t exptab[32];
-    ExpTab et;
-    et.load();
-    // SINGLE: every token of a prefill stack is its own chunk (token y = blockIdx.y at position *pos_dev + y), its
-    // earlier rows all in the cache already (kv_store_kernel), so the workgroup rebuilds only its own row and stores
-    // none.
-    const int h = blockIdx.x, y = blockIdx.y, t = SINGLE ? 0 : y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int pos0 = *pos_dev + (SINGLE ? y : 0), pos = pos0 + t, nrows = pos + 1;
-    if (pos >= ctx || pos0 < 0) {  // uniform: a step past the context touches no cache row
-        if (tid == 0 && h == 0) atomicOr(status, kStatusCtx);
-        return;
-    }
-    const int qd = n_heads * HD, kvd = n_kv * HD, group = n_heads / n_kv, kvh = h / group;
-    if (SINGLE) {  // this token's rows of the projections and of the output
-        q += (size_t)y * qd;
-        k += (size_t)y * kvd;
-        v += (size_t)y * kvd;
-        oq += (size_t)y * qd;
-        od += (size_t)y * (qd / QK);
-        if (of) of += (size_t)y * qd;
-    }
-    QH_PASTAMP(0);
-    // V block b of this head: HD uint4 at vbase + b * kvd (in uint4 units, kvd / 8 per position... see vblock())
-    const uint4* vc4 = reinterpret_cast<const uint4*>(vc);
-    auto vchunk = [&](int blk, int d) { return (size_t)blk * kvd + kvh * HD + d; };  // uint4 index of (block, dim)
-    // K chunk (8 dimensions, 16 bytes) c of position p of this KV head, in 16-byte units: [kv head][HD/8][ctx]
-    auto kchunk = [&](int c, int p) { return ((size_t)kvh * CPR + c) * ctx + p; };
-
-    // this token's q (this head), k and v (its KV head) rows among the chunk's projections
-    const float* qsrc = q + (size_t)t * qd + h * HD;  // row r of k / v: ksrc + r * kvd
-    const float* ksrc = k + kvh * HD;
-    const float* vsrc = v + kvh * HD;
-    const int nk = (t + 1) * HALF, nv = (t + 1) * HD;
-    // q of this head with bias, rotated; keys and values of the chunk's tokens 0..t (model.cpp:183-195, rope
-    // ops_ref.cpp:201-214: a*c - b*s and b*c + a*s with the reference build's contraction fma(a, c, -(b*s)) and
-    // fma(b, c, a*s)). A pair's inputs: the raw values a = row[i], b = row[i + HALF], their biases, cos / sin.
-    struct Pair {
-        float a, b, ba, bb, c, s;
-    };
-    auto load_pair = [&](const float* row, const float* bias, int i, const float* crow) {
-        Pair pr;
-        pr.a = row[i];
-        pr.b = row[i + HALF];
-        pr.ba = bias ? bias[i] : 0.0f;
-        pr.bb = bias ? bias[i + HALF] : 0.0f;
-        pr.c = crow[2 * i];
-        pr.s = crow[2 * i + 1];
-        return pr;
-    };
-    auto rope = [](const Pair& pr, bool has_bias, float& lo, float& hi) {
-        float a = pr.a, b = pr.b;
-        if (has_bias) {
-            a = a + pr.ba;
-            b = b + pr.bb;
-        }
-        lo = __builtin_fmaf(a, pr.c, -(b * pr.s));
-        hi = __builtin_fmaf(b, pr.c, a * pr.s);
-    };
-    const float* bqh = bq ? bq + h * HD : nullptr;
-    const float* bkh = bk ? bk + kvh * HD : nullptr;
-    // Every element this thread rebuilds is loaded before any is used (indices clamped, so every load is
-    // unconditional and the loads are one round trip): K pair elements tid + 256 i and V elements tid + 256 i of the
-    // chunk's rows 0..t. 256 is a multiple of HD, so a thread's elements share their dimension, and its biases.
-    static_assert(256 % HD == 0, "a thread's rebuilt elements share one dimension");
-    constexpr int KPT = kChunk * HALF / 256, VPT = kChunk * HD / 256;  // elements per thread at n = kChunk
-    const int tq = min(tid, HALF - 1);
-    const Pair qp = load_pair(qsrc, bqh, tq, cs + (size_t)pos * HD);
-    const int ik = tid % HALF, iv = tid % HD;
-    const float kba = bkh ? bkh[ik] : 0.0f, kbb = bkh ? bkh[ik + HALF] : 0.0f;
-    const float vb = bv ? bv[kvh * HD + iv] : 0.0f;
-    float ka[KPT], kb[KPT], vv[VPT];
-    float2 kcs[KPT];
-#pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        const int rk = min(tid + 256 * i, nk - 1) / HALF;
-        const float* row = ksrc + (size_t)rk * kvd;
-        ka[i] = row[ik];
-        kb[i] = row[ik + HALF];
-        kcs[i] = *reinterpret_cast<const float2*>(cs + (size_t)(pos0 + rk) * HD + 2 * ik);
-    }
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) vv[i] = vsrc[(size_t)(min(tid + 256 * i, nv - 1) / HD) * kvd + iv];
-    __builtin_amdgcn_sched_barrier(0);
-
-    // This thread's cached K rows for the first score rows (registers) go out behind those (a load waits for every
-    // load issued before it), and their issue, which stalls while the memory pipeline drains, covers the q / k / v
-    // latency. No row read here is written by this launch: K rows stop below pos0.
-    constexpr int kKPre = WPE == 1 ? 3 : 2;  // score rows per thread loaded up front (768 / 512 positions)
-    const int grow = pos0 > 0 ? pos0 - 1 : 0;
-    v4u kpre[kKPre][CPR];
-#pragma unroll
-    for (int r = 0; r < kKPre; ++r) {
-        const uint16_t* kg = kc + (kchunk(0, min(tid + 256 * r, grow)) << 3);
-#pragma unroll
-        for (int i = 0; i < CPR; ++i) kpre[r][i] = ld4(kg + (size_t)i * ctx * 8);
-    }
-    if (tid < HALF) rope(qp, bq != nullptr, qs[tid], qs[tid + HALF]);
-#pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        const int e = tid + 256 * i;
-        if (e < nk) {
-            const int r = e / HALF;
-            float lo, hi;
-            rope(Pair{ka[i], kb[i], kba, kbb, kcs[i].x, kcs[i].y}, bk != nullptr, lo, hi);
-            kloc[r * HD + ik] = f2h(lo);
-            kloc[r * HD + ik + HALF] = f2h(hi);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-        const int e = tid + 256 * i;
-        if (e < nv) vloc[(e / HD) * HD + iv] = f2h(bv ? vv[i] + vb : vv[i]);
-    }
-    et.store(exptab);
-    __syncthreads();
-    QH_PASTAMP(1);
-    if (!SINGLE && h % group == 0)
-        for (int i = tid; i < HD; i += 256) {
-            kc[(kchunk(i >> 3, pos) << 3) + (i & 7)] = kloc[t * HD + i];
-            vc[vchunk(pos / 8, i) * 8 + (pos & 7)] = vloc[t * HD + i];
-        }
-
-    // scores: s = sum_i q_i * k_i as one FMA per element in order, then * scale (model.cpp:122-125)
-    float qv[HD];
-#pragma unroll
-    for (int i = 0; i < HD; ++i) qv[i] = qs[i];
-    const float scale = 1.0f / __builtin_sqrtf((float)HD);
-    float mx = -__builtin_inff();
-    // one dot product: s = fma(q_i, k_i, s) in dimension order
-    auto dot_row = [&](const v4u(&kk)[CPR]) {
-        float sc = 0.0f;
-#pragma unroll
-        for (int i = 0; i < CPR; ++i) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                sc = __builtin_fmaf(qv[i * 8 + 2 * e], h2f((uint16_t)(kk[i][e] & 0xffffu)), sc);
-                sc = __builtin_fmaf(qv[i * 8 + 2 * e + 1], h2f((uint16_t)(kk[i][e] >> 16)), sc);
-            }
-        }
-        return sc;
-    };
-    // the chunk's own rows j >= pos0 (keys in LDS)
-    for (int j = pos0 + tid; j < nrows; j += 256) {
-        v4u kk[CPR];
-        const uint16_t* kl = kloc + (j - pos0) * HD;
-#pragma unroll
-        for (int i = 0; i < CPR; ++i) kk[i] = ld4(kl + i * 8);
-        const float a = dot_row(kk) * scale;
-        att[j] = a;
-        mx = a > mx ? a : mx;
-    }
-    // The first stage's V blocks go straight into LDS (DMA, no registers), in two halves of the whole stage per wave
-    // (clamped onto the last block, whose repeats write the same data): the first once the scores are done and the
-    // second after the exp row (the issue of a half stalls its wave while the memory pipeline drains, so neither
-    // holds up the scores, and the second is issued after the wait that completes the first). Everything is waited
-    // for before the stage is built. Cache blocks stop below pos0: none is written by
-    // this launch (the block holding pos0 carries stale rows from pos0 on, replaced when the stage is built).
-    const int ncb = min((pos0 + 7) / 8, kVBlk);  // cache blocks of the first stage (the last may be partial)
-    constexpr int kDmaPerBlk = HD / 64;          // 1 KB (one wave instruction) per DMA chunk
-    constexpr int kVEarly = kVBlk * kDmaPerBlk / 4;  // DMA chunks per wave
-    auto dma_v = [&](int e0, int e1) {           // chunks wave + 4 e, e in [e0, e1)
-        const int last = max(ncb * kDmaPerBlk - 1, 0);
-#pragma unroll
-        for (int e = e0; e < e1; ++e) {
-            const int c = min(wave + 4 * e, last);
-            lds_dma16_async(vc4 + vchunk(c / kDmaPerBlk, (c % kDmaPerBlk) * 64 + lane), vst + c * 64);
-        }
-    };
-
-    // the cached rows tid + 256 r (registers only), their chains interleaved; stored after the barrier below
-    float sc[kKPre];
-    {
-#pragma unroll
-        for (int r = 0; r < kKPre; ++r)  // uniform: no thread has a cached row tid + 256 r at or past pos0
-            sc[r] = 256 * r < pos0 ? dot_row(kpre[r]) * scale : 0.0f;
-#pragma unroll
-        for (int r = 0; r < kKPre; ++r) {
-            const int j = tid + 256 * r;
-            if (j < pos0) mx = sc[r] > mx ? sc[r] : mx;
-        }
-    }
-    for (int j = tid + 256 * kKPre; j < pos0; j += 256) {  // longer contexts: one row at a time
-        v4u kk[CPR];
-        const uint16_t* kg = kc + (kchunk(0, j) << 3);
-#pragma unroll
-        for (int i = 0; i < CPR; ++i) kk[i] = ld4(kg + (size_t)i * ctx * 8);
-        const float a = dot_row(kk) * scale;
-        att[j] = a;
-        mx = a > mx ? a : mx;
-    }
-    // the maximum does not depend on the order of comparison
-    QH_PASTAMP(2);
-    mx = wave_max_sel(mx);
-    if (lane == 0) red[wave] = mx;
-    dma_v(0, kVEarly / 2);
-#pragma unroll
-    for (int r = 0; r < kKPre; ++r) {
-        const int j = tid + 256 * r;
-        if (j < pos0) att[j] = sc[r];
-    }
-    __syncthreads();
-    mx = red[0];
-    for (int w = 1; w < 4; ++w) mx = red[w] > mx ? red[w] : mx;
-    QH_PASTAMP(3);
-    // exp, kept in LDS, with each lane's exact partial sums below the segment starts
-    const bool seg = nrows >= 128;  // uniform; shorter rows keep the single chain
-    const int Ls = (nrows / 4) & ~15;
-    const Segs4 sg{(nrows - 3 * Ls) & ~15, Ls, nrows};
-    double p1 = 0.0, p2 = 0.0, p3 = 0.0;
-    for (int j = tid; j < nrows; j += 256) {
-        const float e = dev_expf(att[j] - mx, exptab);
-        att[j] = e;
-        p1 += j < sg.start(1) ? (double)e : 0.0;
-        p2 += j < sg.start(2) ? (double)e : 0.0;
-        p3 += j < sg.start(3) ? (double)e : 0.0;
-    }
-    QH_PASTAMP(4);
-    __shared__ SegShared ssh;
-    if (seg) seg_partials(ssh, p1, p2, p3);
-    __builtin_amdgcn_s_waitcnt(0);  // the first half of the V DMA
-    dma_v(kVEarly / 2, kVEarly);
-    __syncthreads();
-    // softmax sum in position order (ops_ref.cpp:220-224)
-    auto add = [](float acc, float a) { return acc + a; };
-    float sum;
-    if (seg) {
-        // segments read as LDS broadcasts (through scalar loads of a global copy written just before, the sum of
-        // 512 positions took 2.3 us against 1.4 us)
-        sum = seg_chain_run(ssh, [&](int k, float s0) { return lds_chain(att + sg.start(k), sg.len(k), add, s0); });
-    } else {
-        __syncthreads();
-        if (tid == 0) sum_sh = lds_chain(att, nrows, add);
-        __syncthreads();
-        sum = sum_sh;
-    }
-    QH_PASTAMP(5);
-    const float inv = 1.0f / sum;
-    for (int j = tid; j < nrows; j += 256) {
-        att[j] = att[j] * inv;
-    }
-    // the V DMA is complete before the barrier; then the chunk's rows that fall inside
-    // the first stage are written over the DMA's blocks
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    uint16_t* vst16 = reinterpret_cast<uint16_t*>(vst);
-    {
-        const int s1 = min(nrows, kVRows);
-        for (int e = tid; e < (s1 - pos0) * HD; e += 256) {  // empty when pos0 >= kVRows
-            const int r = pos0 + e / HD, d = e % HD;
-            vst16[((r >> 3) * HD + d) * 8 + (r & 7)] = vloc[(r - pos0) * HD + d];
-        }
-        __syncthreads();
-    }
-    QH_PASTAMP(6);
-
-    // out_i = sum_j a_j * v_ji, one FMA per position in order (model.cpp:131-135): thread i per dimension, over
-    // the rows of each LDS stage. The weights are broadcast LDS reads of att (every lane the same address), so a
-    // batch of 32 positions is 4 V reads, 8 weight reads and 32 FMAs, the next batch's reads in flight while one is
-    // consumed. (With scalar operands from a global copy of the weights, written just before, the first stage's
-    // chain ran 1.4x slower at two workgroups per CU.) V reads past the stage stay inside its padding, weight reads
-    // inside att's padding.
-    // Past the first stage, the threads without a dimension load the next stage's cache blocks into registers while
-    // the chain runs (kPreload: at most 12 16-byte units each), so only LDS stores stand between two stages.
-    constexpr int kLoaders = 256 - HD, kPre = (kVBlk * HD + kLoaders - 1) / kLoaders;
-    constexpr bool kPreload = kPre <= 12;
-    uint4 nxt[kPreload ? kPre : 1];
-    float acc = 0.0f;
-    for (int s0 = 0;;) {
-        const int se = min(nrows, s0 + kVRows);
-        if (kPreload && tid >= HD && se < nrows) {  // uniform per wave; pos0 >= 1 here (a second stage)
-            const int nb8 = (min(nrows, se + kVRows) - se + 7) / 8, lastc = (pos0 - 1) / 8;
-#pragma unroll
-            for (int u = 0; u < kPre; ++u) {
-                const int c = tid - HD + kLoaders * u, blk = se / 8 + c / HD, d = c % HD;
-                const uint4 x = vc4[vchunk(min(blk, lastc), d)];
-                nxt[u] = c < nb8 * HD && blk * 8 < pos0 ? x : make_uint4(0u, 0u, 0u, 0u);
-            }
-        }
-        if (tid < HD) {
-            // The weights are LDS broadcast reads of att (one 16-byte read gives every lane 4 weights), a batch
-            // ahead of the chain.
-            const float4* ap = reinterpret_cast<const float4*>(att + s0);  // s0 is a multiple of 32
-            auto ldv = [&](uint4(&vv)[4], float4(&w)[8], int jr) {  // rows s0 + jr .. + 31 (jr % 32 == 0)
-                const uint4* vp = vst + (jr >> 3) * HD + tid;
-#pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) vv[q4] = vp[q4 * HD];
-#pragma unroll
-                for (int q = 0; q < 8; ++q) w[q] = ap[jr / 4 + q];
-            };
-            auto use = [&](const uint4(&vv)[4], const float4(&w)[8], int cnt) {
-#pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) {
-                    const uint32_t v[4] = {vv[q4].x, vv[q4].y, vv[q4].z, vv[q4].w};
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int k = 8 * q4 + e;
-                        const float4 wq = w[k >> 2];
-                        const float wk = (k & 3) == 0 ? wq.x : (k & 3) == 1 ? wq.y : (k & 3) == 2 ? wq.z : wq.w;
-                        if (k < cnt)
-                            acc = __builtin_fmaf(wk, h2f((uint16_t)(e & 1 ? v[e >> 1] >> 16 : v[e >> 1] & 0xffffu)),
-                                                 acc);
-                    }
-                }
-            };
-            const int n = se - s0;
-            uint4 vA[4], vB[4];
-            float4 wA[8], wB[8];
-            // sched_barrier keeps each batch's reads ahead of the chain steps they overlap (the scheduler would sink
-            // them next to their first use)
-            ldv(vA, wA, 0);
-            int jr = 0;
-#pragma unroll 1
-            for (; jr + 64 <= n; jr += 64) {
-                ldv(vB, wB, jr + 32);
-                __builtin_amdgcn_sched_barrier(0);
-                use(vA, wA, 32);
-                ldv(vA, wA, jr + 64);
-                __builtin_amdgcn_sched_barrier(0);
-                use(vB, wB, 32);
-            }
-            if (jr + 32 <= n) {
-                ldv(vB, wB, jr + 32);
-                __builtin_amdgcn_sched_barrier(0);
-                use(vA, wA, 32);
-                use(vB, wB, n - jr - 32);
-            } else {
-                use(vA, wA, n - jr);
-            }
-        }
-        s0 = se;
-        if (s0 >= nrows) break;
-        __syncthreads();  // the stage is consumed; load rows [s0, min(nrows, s0 + kVRows)) (s0 % 8 == 0)
-        const int sn = min(nrows, s0 + kVRows);
-        const int nb8 = (sn - s0 + 7) / 8;
-        if constexpr (kPreload) {
-            if (tid >= HD) {
-#pragma unroll
-                for (int u = 0; u < kPre; ++u) {
-                    const int c = tid - HD + kLoaders * u;
-                    if (c < nb8 * HD) vst[c] = nxt[u];
-                }
-            }
-        } else {
-            for (int c = tid; c < nb8 * HD; c += 256) {  // whole cache blocks; the chunk's rows are written after
-                const int blk = s0 / 8 + c / HD, d = c % HD;
-                vst[c] = blk * 8 < pos0 ? vc4[vchunk(blk, d)] : make_uint4(0u, 0u, 0u, 0u);
-            }
-        }
-        __syncthreads();
-        for (int e = tid; e < (sn - max(s0, pos0)) * HD; e += 256) {
-            const int r = max(s0, pos0) + e / HD, d = e % HD;
-            vst16[(((r - s0) >> 3) * HD + d) * 8 + (r & 7)] = vloc[(r - pos0) * HD + d];
-        }
-        __syncthreads();
-    }
-    QH_PASTAMP(7);
-    if (tid < HD) {  // quantize_q8 of the attention output, two 32-blocks per 64 dimensions
-        const int col = h * HD + (tid & ~31);
-        if (of) of[(size_t)t * qd + h * HD + tid] = acc;  // the f32 input of an unquantized o projection
-        quant_block32(acc, oq + (size_t)t * qd + col, od + (size_t)t * (qd / QK) + col / QK);
-    }
-}
-
 // The f16 cache rows of n tokens at positions *pos_dev .. + n - 1 (a prefill stack) from their projections k / v
 // ([n][n_kv * HD]): bias, RoPE as a*c - b*s and b*c + a*s with the reference build's contraction
 // (fma(a, c, -(b*s)), fma(b, c, a*s)), rounded to f16, exactly what attention_kernel rebuilds and stores
@@ -1179,194 +303,6 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const float* __restrict__
     for (int e = tid; e < kvd; e += 256) {
         const float x = v[(size_t)t * kvd + e];
         vc[((size_t)(pos / 8) * kvd + e) * 8 + (pos & 7)] = f2h(bv ? x + bv[e] : x);
-    }
-}
-
-// Attention of a prefill stack at head_dim 64 with kStackTok consecutive tokens of one query head per workgroup, once
-// kv_store_kernel has stored every row of the stack, so the workgroup rebuilds nothing and its tokens share the K and
-// V rows it reads: positions *pos_dev + y0 .. + kStackTok - 1 (y0 = kStackTok * blockIdx.y, tokens below n), all
-// below kStackCtx. The same arithmetic and order as attention_kernel for each token (model.cpp:115-137,
-// ops_ref.cpp:216-226): q with bias and RoPE in f32; wave i takes token i: its q as 64 scalar operands, lane l
-// scores cached rows l, l + 64, ... up to the token's row count (s = fma(q_i, k_i, s) in dimension order, the f16 key
-// as a mixed-precision operand, then * 1/sqrt(64)), the next row's key loaded while a row is scored; the maximum over
-// the wave; glibc expf; the softmax sum in position order, its normalisation, and the weighted V chain over V rows
-// staged in LDS (lane d for dimension d, the weights as LDS broadcast reads), the four tokens' chains on four SIMDs
-// at once. The V stages' loads are issued a stage ahead (the first at the start), so their latency hides under the
-// scores and the previous stage's chains. The output is quantized per 32-block. Its LDS holds two workgroups per CU,
-// so the register budget is that of two waves per SIMD.
-constexpr int kStackTok = 4;
-constexpr int kStackCtx = 1024;
-template <int HD>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void attention_stack_kernel(
-    const float* __restrict__ q, const float* __restrict__ bq, const float* __restrict__ cs,
-    const int* __restrict__ pos_dev, int n, int ctx, int n_heads, int n_kv, const uint16_t* __restrict__ kc,
-    const uint16_t* __restrict__ vc, int8_t* __restrict__ oq, float* __restrict__ od, int* __restrict__ status,
-    float* __restrict__ of) {
-    static_assert(HD == 64, "a lane per dimension");
-    constexpr int HALF = HD / 2, CPR = HD / 8, NTK = kStackTok;
-    constexpr int kVRows = 256, kVBlk = kVRows / 8;  // V rows per LDS stage (32 KB)
-    constexpr int kVPer = kVBlk * HD / 256;          // 16-byte V units per thread and stage
-    __shared__ __align__(16) float att[NTK][kStackCtx + kChainPad];
-    __shared__ __align__(16) uint4 vst[(kVBlk + 4) * HD];  // [block][dim] -> 8 rows; 4 blocks of read padding
-    __shared__ __align__(16) float qs[NTK][HD];
-    __shared__ uint64_t exptab[32];
-    ExpTab et;
-    et.load();
-    // groups in reverse order: the longest (the stack's last tokens) are dispatched first, the short ones fill in
-    const int h = blockIdx.x, y0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * NTK, tid = threadIdx.x, lane = tid & 63,
-              wave = tid >> 6;
-    const int nt = min(NTK, n - y0);  // tokens of this workgroup (uniform)
-    const int base = *pos_dev + y0;   // position of token 0
-    const int nmax = base + nt;       // rows of the last token
-    if (base < 0 || nmax > ctx || nmax > kStackCtx) {  // uniform; the host launches this only within both limits
-        if (tid == 0) atomicOr(status, kStatusCtx);
-        return;
-    }
-    const int qd = n_heads * HD, kvd = n_kv * HD, group = n_heads / n_kv, kvh = h / group;
-    auto kchunk = [&](int c, int p) { return ((size_t)kvh * CPR + c) * ctx + p; };
-    auto vchunk = [&](int blk, int d) { return (size_t)blk * kvd + kvh * HD + d; };
-    const uint4* vc4 = reinterpret_cast<const uint4*>(vc);
-    // V units of the stage at s0 (whole cache blocks of 8 positions below nmax) into registers, then into vst
-    v4u vreg[kVPer];
-    auto vload = [&](int s0) {  // units past the stage's blocks: re-reads, never stored
-        const int nb8 = (min(nmax, s0 + kVRows) - s0 + 7) / 8;
-#pragma unroll
-        for (int k = 0; k < kVPer; ++k) {
-            const int c = min(tid + 256 * k, nb8 * HD - 1);
-            vreg[k] = ld4(vc4 + vchunk(s0 / 8 + c / HD, c % HD));
-        }
-    };
-    auto vput = [&]() {  // the whole stage area (rows past the stage: never read)
-#pragma unroll
-        for (int k = 0; k < kVPer; ++k) *reinterpret_cast<v4u*>(&vst[tid + 256 * k]) = vreg[k];
-    };
-    vload(0);
-    // q of token `wave` (lanes 0-31: one rotated pair each), with bias (model.cpp:183-195, ops_ref.cpp:201-214)
-    if (wave < nt && lane < HALF) {
-        const float* src = q + (size_t)(y0 + wave) * qd + h * HD;
-        const float* crow = cs + (size_t)(base + wave) * HD;
-        float a = src[lane], b = src[lane + HALF];
-        if (bq) {
-            a = a + bq[h * HD + lane];
-            b = b + bq[h * HD + lane + HALF];
-        }
-        const float c = crow[2 * lane], sn = crow[2 * lane + 1];
-        qs[wave][lane] = __builtin_fmaf(a, c, -(b * sn));
-        qs[wave][lane + HALF] = __builtin_fmaf(b, c, a * sn);
-    }
-    et.store(exptab);
-    __syncthreads();
-
-    // wave tk: token tk's scores, maximum, exponentials, softmax sum in position order (ops_ref.cpp:220-224) and
-    // normalisation, all within the wave (its rows of att are its own)
-    const int tk = wave, nrows = base + tk + 1;
-    if (tk < nt) {
-        const float scale = 1.0f / __builtin_sqrtf((float)HD);
-        const float qv = qs[tk][lane];
-        float qsg[HD];  // q_i, wave-uniform
-#pragma unroll
-        for (int d = 0; d < HD; ++d) qsg[d] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, qv), d));
-        float mx = -__builtin_inff();
-        v4u kA[CPR], kB[CPR];
-        auto kload = [&](v4u(&kk)[CPR], int j) {  // row j's key, clamped to the token's last row
-            const uint16_t* kg = kc + (kchunk(0, min(j, nrows - 1)) << 3);
-#pragma unroll
-            for (int c = 0; c < CPR; ++c) kk[c] = ld4(kg + (size_t)c * ctx * 8);
-        };
-        auto score = [&](const v4u(&kk)[CPR], int j) {
-            float sc = 0.0f;
-#pragma unroll
-            for (int c = 0; c < CPR; ++c)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    sc = __builtin_fmaf(qsg[8 * c + 2 * e], h2f((uint16_t)(kk[c][e] & 0xffffu)), sc);
-                    sc = __builtin_fmaf(qsg[8 * c + 2 * e + 1], h2f((uint16_t)(kk[c][e] >> 16)), sc);
-                }
-            if (j < nrows) {
-                const float a = sc * scale;
-                att[tk][j] = a;
-                mx = a > mx ? a : mx;
-            }
-        };
-        kload(kA, lane);
-        int j0 = 0;
-        for (; j0 + 64 < nrows; j0 += 128) {
-            kload(kB, j0 + 64 + lane);
-            score(kA, j0 + lane);
-            kload(kA, j0 + 128 + lane);
-            score(kB, j0 + 64 + lane);
-        }
-        if (j0 < nrows) score(kA, j0 + lane);
-        mx = wave_max_sel(mx);  // the maximum does not depend on the order of comparison
-        __builtin_amdgcn_wave_barrier();
-        for (int j = lane; j < nrows; j += 64) att[tk][j] = dev_expf(att[tk][j] - mx, exptab);
-        __builtin_amdgcn_wave_barrier();
-        const float sum = lds_chain(att[tk], nrows, [](float acc, float a) { return acc + a; });
-        const float inv = 1.0f / sum;
-        for (int j = lane; j < nrows; j += 64) att[tk][j] = att[tk][j] * inv;
-    }
-    // out_i = sum_j a_j * v_ji, one FMA per position in order (model.cpp:131-135): wave i, lane d, over the rows of
-    // each V stage (whole cache blocks of 8 positions; rows past a token's count are never used)
-    float acc = 0.0f;
-    for (int s0 = 0; s0 < nmax; s0 += kVRows) {
-        const int sn = min(nmax, s0 + kVRows);
-        __syncthreads();  // the previous stage is consumed (and, for the first, the normalised rows are written)
-        vput();
-        if (s0 + kVRows < nmax) vload(s0 + kVRows);  // the next stage's loads run under this stage's chains
-        __syncthreads();
-        if (tk < nt && s0 < nrows) {
-            const int n_ = min(nrows, sn) - s0;
-            const float4* ap = reinterpret_cast<const float4*>(lane_ptr(att[tk] + s0));  // s0 % 32 == 0
-            auto ldv = [&](uint4(&vv)[4], float4(&w)[8], int jr) {  // rows s0 + jr .. + 31 (jr % 32 == 0)
-                const uint4* vp = vst + (jr >> 3) * HD + lane;
-#pragma unroll
-                for (int q4i = 0; q4i < 4; ++q4i) vv[q4i] = vp[q4i * HD];
-#pragma unroll
-                for (int qi = 0; qi < 8; ++qi) w[qi] = ap[jr / 4 + qi];
-            };
-            auto use = [&](const uint4(&vv)[4], const float4(&w)[8], int cnt) {
-#pragma unroll
-                for (int q4i = 0; q4i < 4; ++q4i) {
-                    const uint32_t vw[4] = {vv[q4i].x, vv[q4i].y, vv[q4i].z, vv[q4i].w};
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int kx = 8 * q4i + e;
-                        const float4 wq = w[kx >> 2];
-                        const float wk = (kx & 3) == 0 ? wq.x : (kx & 3) == 1 ? wq.y : (kx & 3) == 2 ? wq.z : wq.w;
-                        if (kx < cnt)
-                            acc = __builtin_fmaf(wk, h2f((uint16_t)(e & 1 ? vw[e >> 1] >> 16 : vw[e >> 1] & 0xffffu)),
-                                                 acc);
-                    }
-                }
-            };
-            uint4 vA[4], vB[4];
-            float4 wA[8], wB[8];
-            ldv(vA, wA, 0);
-            int jr = 0;
-#pragma unroll 1
-            for (; jr + 64 <= n_; jr += 64) {
-                ldv(vB, wB, jr + 32);
-                __builtin_amdgcn_sched_barrier(0);
-                use(vA, wA, 32);
-                ldv(vA, wA, jr + 64);
-                __builtin_amdgcn_sched_barrier(0);
-                use(vB, wB, 32);
-            }
-            if (jr + 32 <= n_) {
-                ldv(vB, wB, jr + 32);
-                __builtin_amdgcn_sched_barrier(0);
-                use(vA, wA, 32);
-                use(vB, wB, n_ - jr - 32);
-            } else {
-                use(vA, wA, n_ - jr);
-            }
-        }
-    }
-    if (tk < nt) {  // quantize_q8 of the output, two 32-blocks per 64 dimensions
-        const size_t row = (size_t)(y0 + tk) * qd;
-        const int col = h * HD + (lane & ~31);
-        if (of) of[row + h * HD + lane] = acc;
-        quant_block32(acc, oq + row + col, od + row / QK + col / QK);
     }
 }
 
@@ -2756,8 +1692,6 @@ bool few_workgroups(const qh_model_desc& hp, int n, int pos0) {
     return w <= cus && rows <= 2700;
 }
 
-hipError_t attention_few(Decoder* d, int l, int n, uint16_t* kc, uint16_t* vc, hipStream_t s);
-
 // Attention of a prefill stack of n > kChunk tokens at positions *d->pos ..: the f16 cache rows of every token of the
 // stack first (kv_store_kernel), then the stack's (token, head) pairs together (launch_attention_stack), or, where those
 // are few, one workgroup per head and token (each its own chunk, every earlier row read from the cache) or four tokens.
@@ -2774,7 +1708,10 @@ hipError_t attention_stack(Decoder* d, int l, int n, hipStream_t s) {
                   d->cs, d->pos, hp.ctx_len, hp.n_kv_heads, kc, vc);
     QH_TRY(hipGetLastError());
     const int pos0 = d->stack_end - n;
-    if (few_workgroups(hp, n, pos0)) return attention_few(d, l, n, kc, vc, s);
+    if (few_workgroups(hp, n, pos0))
+        return launch_attention_few({d->q, d->k, d->v, bias(d, l, L_BQ), bias(d, l, L_BK), bias(d, l, L_BV), d->cs, d->pos,
+                                     n, hp.ctx_len, hp.n_heads, hp.n_kv_heads, kc, vc, d->qb, d->db, d->status, d->fb},
+                                    hp.head_dim, d->stack_end, s);
     AttnStack a{};
     a.q = d->q;
     a.bq = bias(d, l, L_BQ);
@@ -3261,30 +2198,5 @@ hipError_t decoder_set_sampler(Decoder* d, const qh_sampler_params* p, uint64_t 
     const uint64_t st = seed | 1u;  // Sampler's constructor (sampler.cpp:10-13)
     return hipMemcpy(d->rng, &st, sizeof st, hipMemcpyHostToDevice);
 }
-
-namespace {
-
-// A stack of few workgroups (few_workgroups), its cache rows stored. Last in the file, its kernels templates, so that the
-// kernels of a decode step keep their places in the code: behind these kernels 16 steps of two layers at position 3,500
-// took 1,915 us, not 1,893.
-hipError_t attention_few(Decoder* d, int l, int n, uint16_t* kc, uint16_t* vc, hipStream_t s) {
-    const qh_model_desc& hp = d->hp;
-    const dim3 grid(hp.n_heads, n);
-    if (hp.head_dim == 64 && d->stack_end <= kStackCtx)
-        qh_launch((attention_stack_kernel<64>), dim3(hp.n_heads, (n + kStackTok - 1) / kStackTok), dim3(256), 0, s, d->q,
-                  bias(d, l, L_BQ), d->cs, d->pos, n, hp.ctx_len, hp.n_heads, hp.n_kv_heads, kc, vc, d->qb, d->db,
-                  d->status, d->fb);
-    else if (hp.head_dim == 64)
-        qh_launch((attention_kernel<64, 2, true>), grid, dim3(256), 0, s, d->q, d->k, d->v, bias(d, l, L_BQ),
-                  bias(d, l, L_BK), bias(d, l, L_BV), d->cs, d->pos, hp.ctx_len, hp.n_heads, hp.n_kv_heads, kc, vc, d->qb,
-                  d->db, d->status, d->fb);
-    else
-        qh_launch((attention_kernel<128, 1, true>), grid, dim3(256), 0, s, d->q, d->k, d->v, bias(d, l, L_BQ),
-                  bias(d, l, L_BK), bias(d, l, L_BV), d->cs, d->pos, hp.ctx_len, hp.n_heads, hp.n_kv_heads, kc, vc, d->qb,
-                  d->db, d->status, d->fb);
-    return hipGetLastError();
-}
-
-}  // namespace
 
 }  // namespace qh

@@ -191,6 +191,21 @@ constexpr size_t kAttnWsBytes = (size_t)256 << 20;
 size_t attn_stack_ws_bytes(int n_heads, int n_kv, int ctx, int tokens, size_t* least_bytes);
 hipError_t launch_attention_stack(AttnStack a, int head_dim, float* ws, size_t ws_bytes, hipStream_t s);
 
+// The same for a stack of few workgroups (qh_attn_few.hip): its projections (without bias or RoPE), *pos its first
+// position, rows the last token's; one workgroup per query head and kStackTok tokens up to kStackCtx rows at head_dim 64.
+struct AttnFew {
+    const float *q, *k, *v, *bq, *bk, *bv, *cs;
+    const int* pos;
+    int n, ctx, n_heads, n_kv;
+    uint16_t *kc, *vc;
+    int8_t* oq;
+    float* od;
+    int* status;
+    float* of;
+};
+constexpr int kStackTok = 4, kStackCtx = 1024;
+hipError_t launch_attention_few(const AttnFew& a, int head_dim, int rows, hipStream_t s);
+
 // GPU-resident decoder (qh_decoder.hip). Tensors in qh_decoder_create order; all sizes validated by the caller.
 struct Decoder;
 int decoder_create(const qh_model_desc* hp, const qh_tensor* tensors, int n_tensors, Decoder** out);
