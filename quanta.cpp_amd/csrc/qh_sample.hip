@@ -262,28 +262,29 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
             strided_bound();
             filter();
         }
-    } else if (n > kThreads && (!rows || k > 64)) {
-        strided_bound();
-        filter();
-    } else {  // the k-th largest of each wave's 64 candidates (when k <= 64)
-        const int i = wave * 64 + lane;
-        const uint64_t a = i < n ? key_of(i) : 0ull;
-        int rank = 0;
-        const int lo = (int)(uint32_t)a, hi = (int)(uint32_t)(a >> 32);
-        for (int j = 0; j < 64; ++j) {
-            const uint64_t kj = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, j) << 32) |
-                                (uint64_t)(uint32_t)__builtin_amdgcn_readlane(lo, j);
-            rank += kj > a ? 1 : 0;
-        }
-        const uint64_t b = (a != 0 && rank == k - 1) ? a : 0ull;
-        const uint64_t bw = wave_max_u64(b);
-        if (lane == 0) wbound[wave] = bw;
-        if (tid == 0) pool_n = 0;
-        __syncthreads();
-        thr = wbound[0];
+    } else {
+        if (n > kThreads && (!rows || k > 64)) {
+            strided_bound();
+        } else {  // the k-th largest of each wave's 64 candidates (when k <= 64)
+            const int i = wave * 64 + lane;
+            const uint64_t a = i < n ? key_of(i) : 0ull;
+            int rank = 0;
+            const int lo = (int)(uint32_t)a, hi = (int)(uint32_t)(a >> 32);
+            for (int j = 0; j < 64; ++j) {
+                const uint64_t kj = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, j) << 32) |
+                                    (uint64_t)(uint32_t)__builtin_amdgcn_readlane(lo, j);
+                rank += kj > a ? 1 : 0;
+            }
+            const uint64_t b = (a != 0 && rank == k - 1) ? a : 0ull;
+            const uint64_t bw = wave_max_u64(b);
+            if (lane == 0) wbound[wave] = bw;
+            if (tid == 0) pool_n = 0;
+            __syncthreads();
+            thr = wbound[0];
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) thr = wbound[w] > thr ? wbound[w] : thr;
-        filter();
+            for (int w = 1; w < kWaves; ++w) thr = wbound[w] > thr ? wbound[w] : thr;
+        }
+        filter();  // one copy of it: the one workgroup's time is latency, of its instructions' first reads too
     }
     const int count = pool_n;
     if (count == 0) {  // uniform; no candidate (an empty row list)
