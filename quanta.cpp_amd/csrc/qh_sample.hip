@@ -257,7 +257,9 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
             }
         }
         __syncthreads();
-        if (pool_n > kPool) {  // uniform; logits crowded into few groups: the bound over strided candidates instead
+        // uniform; logits crowded into few groups all the same (a slow wave along 151,936 ids, top-k 128: 105 us, 85 in one
+        // workgroup alone): the bound over strided candidates instead
+        if (pool_n > kPool) {
             __syncthreads();
             strided_bound();
             filter();
